@@ -1303,15 +1303,17 @@ extern "C" int mlgi_autotune(mlgi_context* c, mlgi_frame_desc* frame, int32_t mi
 
 struct mlgi_scene_device {
   mlgi_context* ctx = nullptr;
-  mlgi_scene_impl::Node4* nodes4 = nullptr;
+  mlgi_scene_impl::Node8* nodes = nullptr;
   mlgi_scene_impl::TriGeo* geo = nullptr;
   mlgi_scene_impl::Tri* tris = nullptr;
   int* order = nullptr;
   double* cdf = nullptr;  // running triangle areas (point sampling)
   double total_area = 0.0;
-  int n_nodes4 = 0, n_tris = 0;
+  int n_nodes = 0, n_tris = 0;
+  float lo[3], hi[3];  // the scene's box
   mlgi_scene_impl::SceneView view() const {
-    return mlgi_scene_impl::SceneView{nodes4, geo, tris, order, n_nodes4, n_tris};
+    return mlgi_scene_impl::SceneView{nodes, geo, tris, order, n_nodes, n_tris,
+                                      {lo[0], lo[1], lo[2]}, {hi[0], hi[1], hi[2]}};
   }
 };
 
@@ -1320,7 +1322,7 @@ extern "C" {
 void mlgi_scene_device_destroy(mlgi_scene_device* d) {
   if (!d) return;
   if (d->ctx) (void)hipStreamSynchronize(d->ctx->stream);
-  (void)hipFree(d->nodes4);
+  (void)hipFree(d->nodes);
   (void)hipFree(d->geo);
   (void)hipFree(d->tris);
   (void)hipFree(d->order);
@@ -1333,17 +1335,19 @@ int mlgi_scene_upload(mlgi_context* c, const mlgi_scene* s, mlgi_scene_device** 
   if (!s || !out) return fail(c, MLGI_ERR_INVALID_ARGUMENT, "scene / out is NULL");
   *out = nullptr;
   const mlgi_scene_impl::SceneView v = mlgi_scene_view(s);
-  if (v.n_nodes4 <= 0 || v.n_tris <= 0) return fail(c, MLGI_ERR_INVALID_ARGUMENT, "empty scene");
+  if (v.n_nodes <= 0 || v.n_tris <= 0) return fail(c, MLGI_ERR_INVALID_ARGUMENT, "empty scene");
   auto* d = new mlgi_scene_device();
   d->ctx = c;
-  d->n_nodes4 = v.n_nodes4;
+  d->n_nodes = v.n_nodes;
   d->n_tris = v.n_tris;
+  std::copy(v.lo, v.lo + 3, d->lo);
+  std::copy(v.hi, v.hi + 3, d->hi);
   auto copy = [&](auto** dst, const auto* src, size_t n, const char* what) {
     int r = hip_check(c, hipMalloc(dst, sizeof(**dst) * n), what);
     if (!r) r = hip_check(c, hipMemcpy(*dst, src, sizeof(**dst) * n, hipMemcpyHostToDevice), what);
     return r;
   };
-  int rc = copy(&d->nodes4, v.nodes4, (size_t)v.n_nodes4, "upload(bvh)");
+  int rc = copy(&d->nodes, v.nodes, (size_t)v.n_nodes, "upload(bvh)");
   if (!rc) rc = copy(&d->geo, v.geo, (size_t)v.n_tris + mlgi_scene_impl::kGeoPad, "upload(triangle geometry)");
   if (!rc) rc = copy(&d->tris, v.tris, (size_t)v.n_tris, "upload(triangles)");
   if (!rc) rc = copy(&d->order, v.order, (size_t)v.n_tris, "upload(order)");

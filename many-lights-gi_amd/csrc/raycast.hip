@@ -1,22 +1,43 @@
-// Device G-buffer / RSM producer: the scene's BVH ray cast on the GPU with
-// the host renderer's double-precision code (scene_trace.hpp), so both write
-// the same texels. Replaces the reference's rasterisation of the G-buffer and
-// RSM (RasterizationStage.cpp and model.frag) for inputs that change per
-// request or per frame. Compiled with -ffp-contract=off like the host
-// renderer.
+// Device G-buffer / RSM producer: the scene's BVH ray cast on the GPU.
+// Replaces the reference's rasterisation of the G-buffer and RSM
+// (RasterizationStage.cpp and model.frag) for inputs that change per request
+// or per frame. Rays, triangle tests and shading are the host renderer's
+// double-precision code (scene_trace.hpp, compiled with -ffp-contract=off
+// like it), and which triangle wins does not depend on the order of the
+// visits, so both write the same texels.
 //
-// Two forms, both single-wave workgroups (a small image then still spreads
-// over every CU) with each ray's traversal stack in LDS (a stack in
-// registers indexed per lane costs a select chain per access):
-//   * one lane per texel, 8x8 texels per wave, for large images;
-//   * four lanes per texel (a quad), 4x4 texels per wave, for images of at
-//     most kQuadRays texels: a 128^2 RSM is 256 waves in the first form, one
-//     per CU, with three of every CU's four SIMDs idle. The quad's lanes
-//     test the four child boxes of an inner node, or the up to four
-//     triangles of a leaf, one each, and exchange the results by DPP quad
-//     broadcasts; every lane then runs the host traversal's ordering
-//     network and leaf-order combination on the same values, so each lane
-//     holds the host's traversal state and the texels are the host's.
+// What bounds it. One traversal per lane spends its time on divergence (an
+// inner step and a leaf step both issue for the whole wave), on the latency
+// of each step's node load, and on the LDS of 64 private stacks (six waves
+// per CU). The rays of a wave's tile are so coherent, though, that one
+// traversal for all of them visits hardly more nodes than one ray's: at 1080p
+// and 40k triangles 23.7 nodes and 11.5 leaves per 8 x 8 tile against 20.8 and
+// 8.9 per ray, for a 128^2 RSM of 160k triangles 22 and 17 per 4 x 4 tile
+// against 21 and 15 (counted on the CPU). So a wave is a packet: it walks the
+// 8-wide tree once, visiting a child if any of its rays enters the child's
+// box before that ray's nearest hit. The current node is wave-uniform, so
+// there is no divergence, and the stack holds one reference per pending child
+// and one entry distance per ray.
+//
+// Boxes are tested in FP32 against node boxes that carry a margin for it
+// (kBoxMargin), which can only visit more nodes; a packet also tests
+// triangles whose box some of its rays miss. Neither changes a texel: every
+// hit is decided by the exact triangle test.
+//
+// Two forms of a packet, in single-wave workgroups:
+//   * 8 x 8 rays, one lane each, for images of 512^2 texels or more: bound by
+//     VALU issue. Node and triangle data are wave-uniform and read through
+//     the scalar cache; each lane tests all children of a node and all
+//     triangles of a leaf for its ray.
+//   * 4 x 4 rays of four lanes each for smaller images, which are bound by
+//     the latency of the steps of their longest packets (a 128^2 RSM is one
+//     wave per SIMD): lane q of a ray's quad tests children q and q + 4 and a
+//     leaf's triangle q, a quarter of the instructions per step.
+// Measured (one traversal per lane or quad over a 4-wide tree -> packets):
+// 1080p G-buffer of 40k triangles 2,234 -> 423 us, 128^2 RSM of 160k
+// 179 -> 61 us, 512^2 RSM 319 -> 115 us. The line between the forms: a 256^2
+// G-buffer takes 77 us in the second form and 136 in the first, a 512^2 one
+// 154 and 145.
 #include "kernels.hpp"
 #include "scene_trace.hpp"
 
@@ -25,108 +46,292 @@ namespace {
 
 using namespace mlgi_scene_impl;
 
-constexpr size_t kQuadRays = size_t(1) << 18;
+constexpr size_t kWideRays = (size_t(1) << 18) - 1;
 
-// Entry i of a ray's stack at base[i * stride].
-struct LdsStack {
-  StackEntry* base;
-  int stride;
-  __device__ void put(int i, const StackEntry& v) { base[i * stride] = v; }
-  __device__ StackEntry get(int i) const { return base[i * stride]; }
+// Pending children whose entry distances are kept; deeper ones are visited
+// without that test. 24 lets the 8 x 8 form run six waves per SIMD, as many as
+// its registers allow (1080p G-buffer, 40k triangles: 423 us, 442 with 32
+// entries); few packets have more pending (19 at most there, 26 in a 128^2
+// RSM of 160k triangles).
+constexpr int kNearStack = 24;
+
+template <int kRays>
+struct PacketLds {
+  float near[kNearStack * kRays];
+  uint32_t ref[kTraceStack];
 };
 
-// A quad's shared stack: lane 0 of the quad writes, all four read.
-struct QuadStack {
-  StackEntry* base;
-  int stride;
-  bool writer;
-  __device__ void put(int i, const StackEntry& v) {
-    if (writer) base[i * stride] = v;
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+__device__ __forceinline__ bool any_lane(bool b) { return __ballot(b) != 0ull; }
+
+// A lane's ray for the FP32 box tests: slab distances lo * i + c along each
+// axis, measured from the ray's entry into the scene's box (`entry`, 0 for a
+// ray that starts inside), and the largest distance still of interest.
+struct BoxRay {
+  float ix, iy, iz, cx, cy, cz, tmax;
+  double entry;
+};
+
+// A bound on the distance to t that is not below it (FP32 rounding, 2^-24).
+__device__ __forceinline__ float box_tmax(double t, double entry) { return (float)(t - entry) * (1.0f + 0x1p-22f); }
+
+__device__ __forceinline__ BoxRay box_ray(const SceneView& s, D3 o, D3 d, double tmax) {
+  BoxRay r;
+  r.entry = 0.0;
+  bool in = true;
+  const bool outside = !(o.x >= s.lo[0] && o.x <= s.hi[0] && o.y >= s.lo[1] && o.y <= s.hi[1] && o.z >= s.lo[2] &&
+                         o.z <= s.hi[2]);
+  if (any_lane(outside)) {
+    // the margin of the scene's box covers the double rounding here
+    double t0;
+    in = box_hit(s.lo, s.hi, o, ray_inverse(d), tmax, &t0);
+    if (outside && in) r.entry = t0;
   }
-  __device__ StackEntry get(int i) const { return base[i * stride]; }
-};
-
-// Value of lane k of this lane's quad (DPP quad_perm [k, k, k, k]). Every lane
-// of a quad is active wherever these are used: a quad's control flow is
-// uniform.
-template <int k>
-__device__ __forceinline__ int quad_lane(int v) {
-  return __builtin_amdgcn_update_dpp(0, v, k | (k << 2) | (k << 4) | (k << 6), 0xF, 0xF, false);
-}
-template <int k>
-__device__ __forceinline__ double quad_lane(double v) {
-  const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
-  const unsigned lo = (unsigned)quad_lane<k>((int)(unsigned)u);
-  const unsigned hi = (unsigned)quad_lane<k>((int)(unsigned)(u >> 32));
-  return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
+  const D3 p = o + d * r.entry;
+  auto inverse = [](double v) {
+    const float f = (float)v;
+    return __builtin_amdgcn_rcpf(fabsf(f) < 1e-18f ? copysignf(1e-18f, f) : f);
+  };
+  r.ix = inverse(d.x);
+  r.iy = inverse(d.y);
+  r.iz = inverse(d.z);
+  r.cx = -((float)p.x * r.ix);
+  r.cy = -((float)p.y * r.iy);
+  r.cz = -((float)p.z * r.iz);
+  r.tmax = in ? box_tmax(tmax, r.entry) : -1.0f;
+  return r;
 }
 
-// trace() of scene_trace.hpp with the four box tests of an inner step and the
-// four triangle tests of a leaf spread over the quad (lane q takes slot q).
-// Leaf: lane q tests against the t at leaf entry; combining in slot order
-// with `hit_k && t_k < t` is the host's sequential test against the running
-// t (t_k itself does not depend on the bound).
-__device__ Hit trace_quad(const SceneView& s, D3 o, D3 d, double tmax, QuadStack& st, int q) {
+// Whether the ray enters the box at most r.tmax away (the distance is
+// clamped to 0 and returned). An unused child's box, a point at 1e18 on every
+// axis, is never hit: its distances are beyond any tmax or negative.
+__device__ __forceinline__ bool box_test(const BoxRay& r, float lx, float ly, float lz, float hx, float hy, float hz,
+                                         float& near) {
+  const float ax = __builtin_fmaf(lx, r.ix, r.cx), bx = __builtin_fmaf(hx, r.ix, r.cx);
+  const float ay = __builtin_fmaf(ly, r.iy, r.cy), by = __builtin_fmaf(hy, r.iy, r.cy);
+  const float az = __builtin_fmaf(lz, r.iz, r.cz), bz = __builtin_fmaf(hz, r.iz, r.cz);
+  near = fmaxf(fmaxf(fmaxf(fminf(ax, bx), fminf(ay, by)), fminf(az, bz)), 0.0f);
+  const float far = fminf(fminf(fminf(fmaxf(ax, bx), fmaxf(ay, by)), fmaxf(az, bz)), r.tmax);
+  return near <= far;
+}
+
+// The packet's direction octant, from its first lane: any octant orders the
+// visits correctly, and the rays of a packet rarely differ.
+__device__ __forceinline__ int packet_octant(D3 d) {
+  const int o = (d.x < 0.0 ? 1 : 0) | (d.y < 0.0 ? 2 : 0) | (d.z < 0.0 ? 4 : 0);
+  return __builtin_amdgcn_readfirstlane(o);
+}
+
+// Pops the nearest pending child that some lane's ray still enters before
+// its nearest hit. `slot` is the lane's ray in the packet. False when none is
+// left.
+template <int kRays>
+__device__ __forceinline__ bool packet_pop(const PacketLds<kRays>& lds, int slot, float tmax, int& sp,
+                                           uint32_t& cur) {
+  wave_sync();  // the stack's entries were written by other lanes
+  while (sp > 0) {
+    --sp;
+    const uint32_t ref = (uint32_t)__builtin_amdgcn_readfirstlane((int)lds.ref[sp]);
+    const float near = sp < kNearStack ? lds.near[sp * kRays + slot] : 0.0f;
+    if (any_lane(near <= tmax)) {
+      cur = ref;
+      return true;
+    }
+  }
+  return false;
+}
+
+// ---------------------------------------------------- 8 x 8 rays, a lane each
+
+template <class T>
+using Uniform = const __attribute__((address_space(4))) T;  // read through the scalar cache
+
+__device__ Hit trace_rays(const SceneView& s, D3 o, D3 d, double tmax, PacketLds<64>& lds) {
+  typedef float f8 __attribute__((ext_vector_type(8)));
+  const int lane = threadIdx.x;
   Hit h{tmax, -1};
-  const D3 inv = ray_inverse(d);
+  BoxRay r = box_ray(s, o, d, tmax);
+  const int oct = packet_octant(d);
+  const int pair = oct < 4 ? oct : oct ^ 7;  // the stored order; reversed for octants 4..7
   int sp = 0;
-  int ref = 0, count = 0;  // the root, an inner node
+  uint32_t cur = 0;  // the root, an inner node
   while (true) {
+    const int count = (int)(cur & 7u);
+    const uint32_t first = cur >> 3;
     if (count == 0) {
-      const float* nf = reinterpret_cast<const float*>(s.nodes4 + ref);
-      const int* ni = reinterpret_cast<const int*>(s.nodes4 + ref);
-      const float lo[3] = {nf[q], nf[4 + q], nf[8 + q]};
-      const float hi[3] = {nf[12 + q], nf[16 + q], nf[20 + q]};
-      const int cref = ni[24 + q], ccnt = ni[28 + q];
-      double tn;
-      const bool hit = box_hit(lo, hi, o, inv, h.t, &tn) && ccnt >= 0;
-      const double key = hit ? tn : kMissed;
-      const int rcq = (cref << 3) | (ccnt & 7);
-      double tk[4] = {quad_lane<0>(key), quad_lane<1>(key), quad_lane<2>(key), quad_lane<3>(key)};
-      int rc[4] = {quad_lane<0>(rcq), quad_lane<1>(rcq), quad_lane<2>(rcq), quad_lane<3>(rcq)};
-      int slot[4] = {0, 1, 2, 3};
-      order_children(tk, slot, rc);
-      for (int i = 3; i >= 1; --i)  // never full (see kTraceStack); checked all the same
-        if (tk[i] < kMissed && sp < kTraceStack) st.put(sp++, StackEntry{rc[i], round_down_f(tk[i])});
-      if (tk[0] < kMissed) {
-        ref = rc[0] >> 3;
-        count = rc[0] & 7;
+      Uniform<f8>* nd = (Uniform<f8>*)(s.nodes + first);
+      Uniform<uint32_t>* words = (Uniform<uint32_t>*)(s.nodes + first);
+      const uint32_t after_lo = words[16 * pair + 7], after_hi = words[16 * pair + 15];
+      float near[8];
+      uint32_t ref[8];
+      uint32_t hits = 0;
+      auto test = [&](int k) {
+        const f8 c = nd[k];
+        ref[k] = __float_as_uint(c[6]);
+        const bool hit = box_test(r, c[0], c[1], c[2], c[3], c[4], c[5], near[k]);
+        if (!hit) near[k] = __builtin_inff();
+        hits |= any_lane(hit) ? 1u << k : 0u;
+      };
+#pragma unroll
+      for (int k = 0; k < 4; ++k) test(k);
+      if (words[8 * 4 + 6] != kNoChild) {
+#pragma unroll
+        for (int k = 4; k < 8; ++k) test(k);
+      }
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        if (!(hits >> k & 1u)) continue;
+        uint32_t after = ((k < 4 ? after_lo : after_hi) >> (8 * (k & 3))) & 0xFFu;
+        if (oct >= 4) after = ~after & ~(1u << k);
+        if ((hits & after) == (hits ^ 1u << k)) {  // the nearest child is visited next
+          cur = ref[k];
+          continue;
+        }
+        const int pos = sp + __builtin_popcount(hits & after);  // < kTraceStack (the build's bound)
+        if (pos < kNearStack) lds.near[pos * 64 + lane] = near[k];
+        if (lane == 0) lds.ref[pos] = ref[k];
+      }
+      if (hits != 0u) {
+        sp += __builtin_popcount(hits) - 1;
         continue;
       }
     } else {
-      const TriGeo g = s.geo[ref + q];  // padded: in bounds for every leaf
-      double th = 0.0;
-      const int hit = (q < count && tri_hit(g, o, d, h.t, &th)) ? 1 : 0;
-      const int hk[4] = {quad_lane<0>(hit), quad_lane<1>(hit), quad_lane<2>(hit), quad_lane<3>(hit)};
-      const double tk[4] = {quad_lane<0>(th), quad_lane<1>(th), quad_lane<2>(th), quad_lane<3>(th)};
-      for (int k = 0; k < 4; ++k) {
-        if (hk[k] && tk[k] < h.t) {
-          h.t = tk[k];
-          h.tri = ref + k;
+      auto load = [&](int k) {
+        Uniform<double>* g = (Uniform<double>*)(s.geo + first + k);
+        return TriGeo{{g[0], g[1], g[2]}, {g[3], g[4], g[5]}, {g[6], g[7], g[8]}};
+      };
+      TriGeo next = load(0);
+      for (int k = 0; k < count; ++k) {
+        const TriGeo t = next;
+        next = load(k + 1);  // requested before this one is tested; padded past the last triangle
+        const TriTerms q = tri_terms(t, o, d);
+        const bool maybe = tri_maybe(q, h.t);
+        if (any_lane(maybe)) {
+          double th;
+          if (maybe && tri_accept(q, h.t, &th) && hit_before(th, (int)first + k, h)) {
+            h.t = th;
+            h.tri = (int)first + k;
+            r.tmax = box_tmax(th, r.entry);
+          }
         }
       }
     }
-    bool more = false;
-    while (sp > 0) {
-      const StackEntry e = st.get(--sp);
-      if (!((double)e.tnear > h.t)) {
-        ref = e.rc >> 3;
-        count = e.rc & 7;
-        more = true;
-        break;
+    if (!packet_pop(lds, lane, r.tmax, sp, cur)) break;
+  }
+  if (h.tri >= 0) h.tri = s.order[h.tri];
+  return h;
+}
+
+struct RayTracer {
+  PacketLds<64>& lds;
+  bool store;
+  __device__ Hit operator()(const SceneView& s, D3 o, D3 d, double tmax) { return trace_rays(s, o, d, tmax, lds); }
+  __device__ bool stores() const { return store; }
+};
+
+// ------------------------------------------------ 4 x 4 rays, four lanes each
+
+// The value of the lane whose number in its quad differs by kXor (1 or 2).
+template <int kXor>
+__device__ __forceinline__ int quad_swap(int v) {
+  constexpr int kCtrl = kXor == 1 ? 0xB1 : 0x4E;  // quad_perm [1,0,3,2], [2,3,0,1]
+  return __builtin_amdgcn_update_dpp(0, v, kCtrl, 0xF, 0xF, false);
+}
+template <int kXor>
+__device__ __forceinline__ double quad_swap(double v) {
+  const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
+  const unsigned lo = (unsigned)quad_swap<kXor>((int)(unsigned)u);
+  const unsigned hi = (unsigned)quad_swap<kXor>((int)(unsigned)(u >> 32));
+  return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
+}
+template <int kXor>
+__device__ __forceinline__ void quad_nearest(Hit& h) {
+  const double t = quad_swap<kXor>(h.t);
+  const int tri = quad_swap<kXor>(h.tri);
+  if (tri >= 0 && hit_before(t, tri, h)) h = Hit{t, tri};
+}
+
+// Bit q set: some ray's lane q has its bit of b set.
+__device__ __forceinline__ uint32_t any_of_quads(unsigned long long b) {
+  uint32_t m = (uint32_t)(b | b >> 32);
+  m |= m >> 16;
+  m |= m >> 8;
+  m |= m >> 4;
+  return m & 15u;
+}
+
+__device__ Hit trace_quads(const SceneView& s, D3 o, D3 d, double tmax, PacketLds<16>& lds) {
+  const int lane = threadIdx.x, q = lane & 3, slot = lane >> 2;
+  Hit h{tmax, -1};  // the same in a quad's lanes
+  BoxRay r = box_ray(s, o, d, tmax);
+  const int oct = packet_octant(d);
+  const int pair = oct < 4 ? oct : oct ^ 7;
+  int sp = 0;
+  uint32_t cur = 0;
+  while (true) {
+    const int count = (int)(cur & 7u);
+    const uint32_t first = cur >> 3;
+    if (count == 0) {
+      const float4* c = reinterpret_cast<const float4*>(s.nodes + first);
+      const float4 a0 = c[2 * q], a1 = c[2 * q + 1], b0 = c[2 * q + 8], b1 = c[2 * q + 9];
+      const uint32_t* words = reinterpret_cast<const uint32_t*>(s.nodes + first);
+      uint32_t after0 = words[16 * pair + 7] >> (8 * q) & 0xFFu, after1 = words[16 * pair + 15] >> (8 * q) & 0xFFu;
+      float near0, near1;
+      const bool hit0 = box_test(r, a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, near0);
+      const bool hit1 = box_test(r, b0.x, b0.y, b0.z, b0.w, b1.x, b1.y, near1);
+      const uint32_t hits = any_of_quads(__ballot(hit0)) | any_of_quads(__ballot(hit1)) << 4;
+      if (oct >= 4) {
+        after0 = ~(after0 | 1u << q);
+        after1 = ~(after1 | 16u << q);
+      }
+      after0 &= hits;
+      after1 &= hits;
+      const bool any0 = hits >> q & 1u, any1 = hits >> q & 16u;
+      const bool top0 = any0 && after0 == (hits ^ 1u << q), top1 = any1 && after1 == (hits ^ 16u << q);
+      const uint32_t ref0 = __float_as_uint(a1.z), ref1 = __float_as_uint(b1.z);
+      // positions below kTraceStack (the build's bound)
+      const int pos0 = sp + __builtin_popcount(after0), pos1 = sp + __builtin_popcount(after1);
+      if (any0 && !top0) {
+        if (pos0 < kNearStack) lds.near[pos0 * 16 + slot] = hit0 ? near0 : __builtin_inff();
+        if (slot == 0) lds.ref[pos0] = ref0;
+      }
+      if (any1 && !top1) {
+        if (pos1 < kNearStack) lds.near[pos1 * 16 + slot] = hit1 ? near1 : __builtin_inff();
+        if (slot == 0) lds.ref[pos1] = ref1;
+      }
+      if (hits != 0u) {  // the nearest child is visited next, without a turn through the stack
+        cur = (uint32_t)__builtin_amdgcn_readlane((int)(top0 ? ref0 : ref1), __builtin_ctzll(__ballot(top0 || top1)));
+        sp += __builtin_popcount(hits) - 1;
+        continue;
+      }
+    } else {
+      const TriGeo g = s.geo[first + q];  // padded: in bounds for every leaf
+      const TriTerms k = tri_terms(g, o, d);
+      const bool maybe = q < count && tri_maybe(k, h.t);
+      if (any_lane(maybe)) {
+        double th;
+        if (maybe && tri_accept(k, h.t, &th) && hit_before(th, (int)first + q, h)) h = Hit{th, (int)first + q};
+        quad_nearest<1>(h);
+        quad_nearest<2>(h);
+        if (h.tri >= 0) r.tmax = box_tmax(h.t, r.entry);
       }
     }
-    if (!more) break;
+    if (!packet_pop(lds, slot, r.tmax, sp, cur)) break;
   }
   if (h.tri >= 0) h.tri = s.order[h.tri];
   return h;
 }
 
 struct QuadTracer {
-  QuadStack st;
-  int q;
-  __device__ Hit operator()(const SceneView& s, D3 o, D3 d, double tmax) { return trace_quad(s, o, d, tmax, st, q); }
-  __device__ bool stores() const { return q == 0; }
+  PacketLds<16>& lds;
+  bool store;
+  __device__ Hit operator()(const SceneView& s, D3 o, D3 d, double tmax) { return trace_quads(s, o, d, tmax, lds); }
+  __device__ bool stores() const { return store; }
 };
 
 template <class Tracer>
@@ -140,34 +345,34 @@ __device__ __forceinline__ void shade(Tracer& tr, const SceneView& s, const RayC
     shade_gbuffer(tr, s, rc, x, y, w, h, a, b);  // depth, normal
 }
 
+// Lanes past the image repeat its last row or column (the whole wave runs the
+// packet) and store nothing.
 __global__ __launch_bounds__(64) void raycast_kernel(SceneView s, RayCam rc, int w, int h, int mode,
                                                       float* __restrict__ a, float* __restrict__ b,
                                                       float* __restrict__ c) {
-  __shared__ StackEntry stack[kTraceStack * 64];
+  __shared__ PacketLds<64> lds;
   const int x = blockIdx.x * 8 + (threadIdx.x & 7);
   const int y = blockIdx.y * 8 + (threadIdx.x >> 3);
-  if (x >= w || y >= h) return;
-  StackTracer<LdsStack> tr{LdsStack{stack + threadIdx.x, 64}};
-  shade(tr, s, rc, x, y, w, h, mode, a, b, c);
+  RayTracer tr{lds, x < w && y < h};
+  shade(tr, s, rc, min(x, w - 1), min(y, h - 1), w, h, mode, a, b, c);
 }
 
 __global__ __launch_bounds__(64) void raycast_quad_kernel(SceneView s, RayCam rc, int w, int h, int mode,
                                                            float* __restrict__ a, float* __restrict__ b,
                                                            float* __restrict__ c) {
-  __shared__ StackEntry stack[kTraceStack * 16];
+  __shared__ PacketLds<16> lds;
   const int q = threadIdx.x & 3, r = threadIdx.x >> 2;
   const int x = blockIdx.x * 4 + (r & 3);
   const int y = blockIdx.y * 4 + (r >> 2);
-  if (x >= w || y >= h) return;  // the whole quad
-  QuadTracer tr{QuadStack{stack + r, 16, q == 0}, q};
-  shade(tr, s, rc, x, y, w, h, mode, a, b, c);
+  QuadTracer tr{lds, q == 0 && x < w && y < h};
+  shade(tr, s, rc, min(x, w - 1), min(y, h - 1), w, h, mode, a, b, c);
 }
 
 }  // namespace
 
 hipError_t launch_raycast(hipStream_t st, const SceneView& s, const RayCam& rc, int w, int h, int rsm,
                           float* a, float* b, float* c) {
-  if ((size_t)w * (size_t)h <= kQuadRays) {
+  if ((size_t)w * (size_t)h <= kWideRays) {
     const dim3 grid((w + 3) / 4, (h + 3) / 4);
     hipLaunchKernelGGL(raycast_quad_kernel, grid, dim3(64), 0, st, s, rc, w, h, rsm, a, b, c);
   } else {

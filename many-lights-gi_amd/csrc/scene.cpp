@@ -35,9 +35,9 @@ struct Rng {
 struct mlgi_scene {
   std::vector<Tri> tris;
   std::vector<int> order;  // BVH leaf order
-  std::vector<Node> nodes;    // binary BVH (build)
-  std::vector<Node4> nodes4;  // 4-wide BVH (traversal)
-  std::vector<TriGeo> geo;    // triangle geometry in leaf order
+  std::vector<Node8> nodes;  // 8-wide BVH
+  std::vector<TriGeo> geo;   // triangle geometry in leaf order
+  float lo[3], hi[3];        // the scene's box, with the nodes' margin
   double area = 0.0;
 };
 
@@ -45,253 +45,288 @@ namespace {
 
 const D3 kDefaultEye = {5.0, 5.0, 9.0};
 
-// Depth of the subtree at node i (the traversal stack must hold it).
-int bvh_depth(const mlgi_scene* s, int i) {
-  const Node& nd = s->nodes[i];
-  if (nd.count > 0) return 1;
-  return 1 + std::max(bvh_depth(s, nd.left), bvh_depth(s, nd.left + 1));
-}
-
-void build_bvh_with(mlgi_scene* s, int sah_depth) {
-  const int n = (int)s->tris.size();
-  s->order.resize(n);
-  for (int i = 0; i < n; ++i) s->order[i] = i;
-  std::vector<D3> cen(n);
-  for (int i = 0; i < n; ++i) cen[i] = (s->tris[i].v0 + s->tris[i].v1 + s->tris[i].v2) * (1.0 / 3.0);
-  s->nodes.clear();
-  s->nodes.reserve(2 * n + 2);
-  struct Item {
-    int node, begin, end, depth;
-  };
-  std::vector<Item> stack;
-  s->nodes.push_back(Node{});
-  // Root split by size: triangles spanning more than a quarter of the scene
-  // (the room's walls) go to their own subtree, so the boxes of the median
-  // splits below stay tight around the small geometry instead of every level
-  // containing a wall (which each ray would then enter).
-  double slo[3] = {1e300, 1e300, 1e300}, shi[3] = {-1e300, -1e300, -1e300};
-  for (const Tri& t : s->tris)
-    for (const D3* v : {&t.v0, &t.v1, &t.v2})
-      for (int k = 0; k < 3; ++k) {
-        slo[k] = std::min(slo[k], comp(*v, k));
-        shi[k] = std::max(shi[k], comp(*v, k));
-      }
-  const double span = std::max(shi[0] - slo[0], std::max(shi[1] - slo[1], shi[2] - slo[2]));
-  auto big = [&](int i) {
-    const Tri& t = s->tris[i];
-    for (int k = 0; k < 3; ++k) {
-      const double lo = std::min(comp(t.v0, k), std::min(comp(t.v1, k), comp(t.v2, k)));
-      const double hi = std::max(comp(t.v0, k), std::max(comp(t.v1, k), comp(t.v2, k)));
-      if (hi - lo > 0.25 * span) return true;
-    }
-    return false;
-  };
-  const int n_big = (int)(std::stable_partition(s->order.begin(), s->order.end(), big) - s->order.begin());
-  if (n_big > 0 && n_big < n && n > 4) {
-    Node root{};
-    for (int k = 0; k < 3; ++k) {
-      root.lo[k] = slo[k];
-      root.hi[k] = shi[k];
-    }
-    root.left = 1;
-    root.count = -1;  // inner node; children: walls (1), the rest (2); axis 0 for the visiting order
-    s->nodes[0] = root;
-    s->nodes.push_back(Node{});
-    s->nodes.push_back(Node{});
-    stack.push_back({1, 0, n_big, 1});
-    stack.push_back({2, n_big, n, 1});
-  } else {
-    stack.push_back({0, 0, n, 0});
-  }
-  while (!stack.empty()) {
-    Item it = stack.back();
-    stack.pop_back();
-    Node nd{};
-    for (int k = 0; k < 3; ++k) {
-      nd.lo[k] = 1e300;
-      nd.hi[k] = -1e300;
-    }
-    double clo[3] = {1e300, 1e300, 1e300}, chi[3] = {-1e300, -1e300, -1e300};
-    for (int i = it.begin; i < it.end; ++i) {
-      const Tri& t = s->tris[s->order[i]];
-      for (const D3* v : {&t.v0, &t.v1, &t.v2})
-        for (int k = 0; k < 3; ++k) {
-          nd.lo[k] = std::min(nd.lo[k], comp(*v, k));
-          nd.hi[k] = std::max(nd.hi[k], comp(*v, k));
-        }
-      for (int k = 0; k < 3; ++k) {
-        clo[k] = std::min(clo[k], comp(cen[s->order[i]], k));
-        chi[k] = std::max(chi[k], comp(cen[s->order[i]], k));
-      }
-    }
-    const int cnt = it.end - it.begin;
-    if (cnt <= 4) {
-      nd.left = it.begin;
-      nd.count = cnt;
-      s->nodes[it.node] = nd;
-      continue;
-    }
-    // Binned surface-area heuristic on the top levels: 16 centroid bins per
-    // axis, the split plane of least (area x count) over both sides. Median
-    // splits below (and where all centroids coincide or a side would be
-    // empty), so the depth stays within sah_depth + log2(n / 4) + 1.
-    constexpr int kBins = 16;
-    int axis = -1, split = -1;
-    double best = 1e300;
-    for (int k = 0; k < 3 && it.depth < sah_depth; ++k) {
-      const double ext = chi[k] - clo[k];
-      if (!(ext > 0.0)) continue;
-      int bc[kBins] = {};
-      double blo[kBins][3], bhi[kBins][3];
-      for (int b = 0; b < kBins; ++b)
-        for (int q = 0; q < 3; ++q) {
-          blo[b][q] = 1e300;
-          bhi[b][q] = -1e300;
-        }
-      for (int i = it.begin; i < it.end; ++i) {
-        const int ti = s->order[i];
-        const int b = std::min(kBins - 1, (int)((comp(cen[ti], k) - clo[k]) / ext * kBins));
-        bc[b]++;
-        const Tri& t = s->tris[ti];
-        for (const D3* v : {&t.v0, &t.v1, &t.v2})
-          for (int q = 0; q < 3; ++q) {
-            blo[b][q] = std::min(blo[b][q], comp(*v, q));
-            bhi[b][q] = std::max(bhi[b][q], comp(*v, q));
-          }
-      }
-      auto area = [](const double* lo, const double* hi) {
-        if (lo[0] > hi[0]) return 0.0;
-        const double x = hi[0] - lo[0], y = hi[1] - lo[1], z = hi[2] - lo[2];
-        return 2.0 * (x * y + y * z + z * x);
-      };
-      double rlo[kBins][3], rhi[kBins][3];
-      int rc[kBins];
-      double alo[3] = {1e300, 1e300, 1e300}, ahi[3] = {-1e300, -1e300, -1e300};
-      int acc = 0;
-      for (int b = kBins - 1; b >= 0; --b) {  // suffix boxes and counts
-        for (int q = 0; q < 3; ++q) {
-          alo[q] = std::min(alo[q], blo[b][q]);
-          ahi[q] = std::max(ahi[q], bhi[b][q]);
-          rlo[b][q] = alo[q];
-          rhi[b][q] = ahi[q];
-        }
-        acc += bc[b];
-        rc[b] = acc;
-      }
-      double llo[3] = {1e300, 1e300, 1e300}, lhi[3] = {-1e300, -1e300, -1e300};
-      int lc = 0;
-      for (int sp = 1; sp < kBins; ++sp) {  // left = bins [0, sp)
-        for (int q = 0; q < 3; ++q) {
-          llo[q] = std::min(llo[q], blo[sp - 1][q]);
-          lhi[q] = std::max(lhi[q], bhi[sp - 1][q]);
-        }
-        lc += bc[sp - 1];
-        if (lc == 0 || rc[sp] == 0) continue;
-        const double cost = area(llo, lhi) * lc + area(rlo[sp], rhi[sp]) * rc[sp];
-        if (cost < best) {
-          best = cost;
-          axis = k;
-          split = sp;
-        }
-      }
-    }
-    int mid = -1;
-    if (axis >= 0) {
-      const double ext = chi[axis] - clo[axis];
-      const int ax = axis, spl = split;
-      const double c0 = clo[axis];
-      mid = (int)(std::stable_partition(s->order.begin() + it.begin, s->order.begin() + it.end,
-                                        [&](int ti) {
-                                          return std::min(kBins - 1, (int)((comp(cen[ti], ax) - c0) / ext * kBins)) <
-                                                 spl;
-                                        }) -
-                  s->order.begin());
-    }
-    if (mid <= it.begin || mid >= it.end) {
-      axis = 0;
-      for (int k = 1; k < 3; ++k)
-        if (chi[k] - clo[k] > chi[axis] - clo[axis]) axis = k;
-      mid = (it.begin + it.end) / 2;
-      std::nth_element(s->order.begin() + it.begin, s->order.begin() + mid, s->order.begin() + it.end,
-                       [&](int a, int b) {
-                         double ca = comp(cen[a], axis), cb = comp(cen[b], axis);
-                         return ca < cb || (ca == cb && a < b);
-                       });
-    }
-    nd.left = (int)s->nodes.size();
-    nd.count = -1 - axis;  // inner node: split axis
-    s->nodes[it.node] = nd;
-    s->nodes.push_back(Node{});
-    s->nodes.push_back(Node{});
-    stack.push_back({nd.left, it.begin, mid, it.depth + 1});
-    stack.push_back({nd.left + 1, mid, it.end, it.depth + 1});
-  }
-}
-
 // Float bounds that contain the double ones.
 float round_up_f(double x) {
   float f = (float)x;
   if ((double)f < x) f = std::nextafter(f, HUGE_VALF);
   return f;
 }
-float round_down_any(double x) {
+float round_down_f(double x) {
   float f = (float)x;
   if ((double)f > x) f = std::nextafter(f, -HUGE_VALF);
   return f;
 }
 
-// 4-wide node of binary node b (an inner node, or a leaf root): its children,
-// each inner child replaced by its own two children, in binary order.
-int collapse(mlgi_scene* s, int b) {
-  const int me = (int)s->nodes4.size();
-  s->nodes4.push_back(Node4{});
-  int slots[4], n = 0;
-  const Node nd = s->nodes[b];
-  if (nd.count > 0) {
-    slots[n++] = b;
+struct Box {
+  float lo[3], hi[3];
+  void clear() {
+    for (int k = 0; k < 3; ++k) lo[k] = HUGE_VALF, hi[k] = -HUGE_VALF;
+  }
+  void add(const float* l, const float* h) {
+    for (int k = 0; k < 3; ++k) {
+      lo[k] = l[k] < lo[k] ? l[k] : lo[k];
+      hi[k] = h[k] > hi[k] ? h[k] : hi[k];
+    }
+  }
+  float area() const {
+    const float x = hi[0] - lo[0], y = hi[1] - lo[1], z = hi[2] - lo[2];
+    return x < 0.0f ? 0.0f : x * y + y * z + z * x;
+  }
+};
+
+// A triangle as the build sees it: its box (floats, rounded outward) and twice
+// its centre.
+struct Prim {
+  float lo[3], hi[3], c[3];
+  int tri;
+};
+
+// The binary tree over prims (reordered into leaf order): binned surface-area
+// splits down to depth sah_depth, median splits below it and wherever no
+// binned split separates; leaves of at most kLeafTris triangles.
+void build_binary(std::vector<Prim>& prims, float span, int sah_depth, std::vector<Node>& nodes) {
+  const int n = (int)prims.size();
+  nodes.clear();
+  nodes.reserve(n + 8);
+  nodes.push_back(Node{});
+  struct Item {
+    int node, begin, end, depth;
+  };
+  std::vector<Item> stack;
+  // Root split by size: triangles spanning more than a quarter of the scene
+  // (the room's walls) go to their own subtree, so the boxes of the splits
+  // below stay tight around the small geometry instead of every level
+  // containing a wall (which each ray would then enter).
+  auto big = [&](const Prim& p) {
+    for (int k = 0; k < 3; ++k)
+      if (p.hi[k] - p.lo[k] > 0.25f * span) return true;
+    return false;
+  };
+  const int n_big = (int)(std::stable_partition(prims.begin(), prims.end(), big) - prims.begin());
+  auto inner = [&](int node, int begin, int mid, int end, int depth) {
+    nodes[node].left = (int)nodes.size();
+    nodes[node].count = 0;
+    const int left = nodes[node].left;
+    nodes.push_back(Node{});
+    nodes.push_back(Node{});
+    stack.push_back({left, begin, mid, depth + 1});
+    stack.push_back({left + 1, mid, end, depth + 1});
+  };
+  if (n_big > 0 && n_big < n && n > kLeafTris) {
+    Box b;
+    b.clear();
+    for (const Prim& p : prims) b.add(p.lo, p.hi);
+    std::copy(b.lo, b.lo + 3, nodes[0].lo);
+    std::copy(b.hi, b.hi + 3, nodes[0].hi);
+    inner(0, 0, n_big, n, 0);
   } else {
-    for (int c : {nd.left, nd.left + 1}) {
-      const Node& cn = s->nodes[c];
-      if (cn.count > 0) {
-        slots[n++] = c;
-      } else {
-        slots[n++] = cn.left;
-        slots[n++] = cn.left + 1;
+    stack.push_back({0, 0, n, 0});
+  }
+  while (!stack.empty()) {
+    const Item it = stack.back();
+    stack.pop_back();
+    const int cnt = it.end - it.begin;
+    Prim* const p0 = prims.data() + it.begin;
+    Box b;
+    b.clear();
+    float clo[3] = {HUGE_VALF, HUGE_VALF, HUGE_VALF}, chi[3] = {-HUGE_VALF, -HUGE_VALF, -HUGE_VALF};
+    for (int i = 0; i < cnt; ++i) {
+      b.add(p0[i].lo, p0[i].hi);
+      for (int k = 0; k < 3; ++k) {
+        clo[k] = std::min(clo[k], p0[i].c[k]);
+        chi[k] = std::max(chi[k], p0[i].c[k]);
       }
     }
-  }
-  Node4 q{};
-  for (int k = 0; k < 4; ++k) {
-    q.ref[k] = 0;
-    q.count[k] = -1;
-    for (int a = 0; a < 3; ++a) q.lo[a][k] = q.hi[a][k] = 0.0f;
-  }
-  for (int k = 0; k < n; ++k) {
-    const Node c = s->nodes[slots[k]];
-    for (int a = 0; a < 3; ++a) {
-      q.lo[a][k] = round_down_any(c.lo[a]);
-      q.hi[a][k] = round_up_f(c.hi[a]);
+    std::copy(b.lo, b.lo + 3, nodes[it.node].lo);
+    std::copy(b.hi, b.hi + 3, nodes[it.node].hi);
+    if (cnt <= kLeafTris) {
+      nodes[it.node].left = it.begin;
+      nodes[it.node].count = cnt;
+      continue;
     }
-    q.ref[k] = c.count > 0 ? c.left : collapse(s, slots[k]);
-    q.count[k] = c.count > 0 ? c.count : 0;
+    // Binned surface-area heuristic: centroid bins per axis (as many as
+    // triangles in small nodes), the plane of least (area x count) over both
+    // sides.
+    constexpr int kBins = 16;
+    const int nb = std::min(kBins, std::max(4, cnt));
+    int axis = -1, split = -1;
+    float scale[3];
+    auto bin_of = [&](const Prim& p, int k) { return std::min(nb - 1, (int)((p.c[k] - clo[k]) * scale[k])); };
+    if (it.depth < sah_depth) {
+      Box bx[3][kBins];
+      int bc[3][kBins];
+      for (int k = 0; k < 3; ++k) {
+        scale[k] = chi[k] > clo[k] ? (float)nb / (chi[k] - clo[k]) : 0.0f;
+        if (!(scale[k] < HUGE_VALF)) scale[k] = 0.0f;
+        for (int q = 0; q < nb; ++q) {
+          bx[k][q].clear();
+          bc[k][q] = 0;
+        }
+      }
+      for (int i = 0; i < cnt; ++i)
+        for (int k = 0; k < 3; ++k) {
+          const int q = bin_of(p0[i], k);
+          bx[k][q].add(p0[i].lo, p0[i].hi);
+          bc[k][q]++;
+        }
+      float best = HUGE_VALF;
+      for (int k = 0; k < 3; ++k) {
+        float right[kBins];  // area x count of bins [q, nb)
+        Box acc;
+        acc.clear();
+        int rc = 0;
+        for (int q = nb - 1; q >= 1; --q) {
+          acc.add(bx[k][q].lo, bx[k][q].hi);
+          rc += bc[k][q];
+          right[q] = acc.area() * (float)rc;
+        }
+        acc.clear();
+        int lc = 0;
+        for (int q = 1; q < nb; ++q) {  // left = bins [0, q)
+          acc.add(bx[k][q - 1].lo, bx[k][q - 1].hi);
+          lc += bc[k][q - 1];
+          if (lc == 0 || lc == cnt) continue;
+          const float cost = acc.area() * (float)lc + right[q];
+          if (cost < best) {
+            best = cost;
+            axis = k;
+            split = q;
+          }
+        }
+      }
+    }
+    int mid = 0;
+    if (axis >= 0) {
+      const int ax = axis, spl = split;
+      mid = (int)(std::partition(p0, p0 + cnt, [&](const Prim& p) { return bin_of(p, ax) < spl; }) - p0);
+    }
+    if (mid <= 0 || mid >= cnt) {
+      axis = 0;
+      for (int k = 1; k < 3; ++k)
+        if (chi[k] - clo[k] > chi[axis] - clo[axis]) axis = k;
+      mid = cnt / 2;
+      std::nth_element(p0, p0 + mid, p0 + cnt, [axis](const Prim& a, const Prim& c) {
+        return a.c[axis] < c.c[axis] || (a.c[axis] == c.c[axis] && a.tri < c.tri);
+      });
+    }
+    inner(it.node, it.begin, it.begin + mid, it.end, it.depth);
   }
-  s->nodes4[me] = q;
-  return me;
 }
 
-// SAH on the top 8 levels; if the tree outgrows the traversal stack, which
-// holds three pending children per 4-wide level and so needs a binary depth
-// of at most 32 (only for far larger scenes than generated here), median
-// splits only, which are ceil(log2(n / 4)) + 2 <= 32 deep. Then the 4-wide
-// tree and the leaf-order triangle geometry.
+// 8-wide node of binary node b: the child of largest area is opened until
+// eight are there (levels: the children of three binary levels, opened
+// whatever their area, which bounds the depth). Returns the most children
+// that can be pending below it (kTraceStack).
+int collapse8(mlgi_scene* s, const std::vector<Node>& bin, int b, float margin, bool levels) {
+  const int me = (int)s->nodes.size();
+  s->nodes.push_back(Node8{});
+  int kid[8] = {b}, depth[8] = {0}, n = 1;
+  auto area = [&](int x) {
+    Box q;
+    std::copy(bin[x].lo, bin[x].lo + 3, q.lo);
+    std::copy(bin[x].hi, bin[x].hi + 3, q.hi);
+    return q.area();
+  };
+  while (n < 8) {
+    int open = -1;
+    float best = -1.0f;
+    for (int k = 0; k < n; ++k) {
+      if (bin[kid[k]].count > 0 || (levels && depth[k] == 3)) continue;
+      const float a = levels ? 8.0f - (float)depth[k] : area(kid[k]);
+      if (a > best) best = a, open = k;
+    }
+    if (open < 0) break;
+    const int left = bin[kid[open]].left;
+    depth[n] = ++depth[open];
+    kid[open] = left;
+    kid[n++] = left + 1;
+  }
+  Node8 q;
+  float centre[8][3];
+  int most = 0;
+  for (int k = 0; k < 8; ++k) {
+    Child8& c = q.c[k];
+    c.after = 0;
+    if (k >= n) {
+      c.ref = kNoChild;
+      // a point no ray reaches: the slab test sorts each axis's two planes, so
+      // an inverted box would count as an endless one
+      for (int a = 0; a < 3; ++a) c.lo[a] = c.hi[a] = 1e18f;
+      continue;
+    }
+    const Node& x = bin[kid[k]];
+    for (int a = 0; a < 3; ++a) {
+      c.lo[a] = round_down_f((double)x.lo[a] - margin);
+      c.hi[a] = round_up_f((double)x.hi[a] + margin);
+      centre[k][a] = 0.5f * x.lo[a] + 0.5f * x.hi[a];
+    }
+    if (x.count > 0) {
+      c.ref = (uint32_t)x.left << 3 | (uint32_t)x.count;
+    } else {
+      c.ref = (uint32_t)s->nodes.size() << 3;
+      most = std::max(most, collapse8(s, bin, kid[k], margin, levels));
+    }
+  }
+  // children by their centres' distance along the octant's diagonal
+  for (int o = 0; o < 4; ++o) {
+    float key[8];
+    for (int k = 0; k < n; ++k) {
+      key[k] = 0.0f;
+      for (int a = 0; a < 3; ++a) key[k] += (o >> a & 1) ? -centre[k][a] : centre[k][a];
+    }
+    uint32_t word[2] = {0, 0};
+    for (int k = 0; k < n; ++k)
+      for (int j = 0; j < n; ++j)
+        if (key[j] > key[k] || (key[j] == key[k] && j > k)) word[k >> 2] |= (1u << j) << (8 * (k & 3));
+    q.c[2 * o].after = word[0];
+    q.c[2 * o + 1].after = word[1];
+  }
+  s->nodes[me] = q;
+  return most + n - 1;
+}
+
+// Binned splits throughout; if the tree could outgrow the traversal stack
+// (only for far larger scenes than generated here), median splits and whole
+// levels: at most 7 pending children for each three binary levels, of which
+// median splits make ceil(log2(n / 4)) + 2 <= 31. Then the triangle geometry
+// in leaf order.
 void build_bvh(mlgi_scene* s) {
-  build_bvh_with(s, 8);
-  if (bvh_depth(s, 0) > 2 * kTraceStack / 3) build_bvh_with(s, 0);
-  s->nodes4.clear();
-  s->nodes4.reserve(s->nodes.size() / 2 + 2);
-  collapse(s, 0);
-  s->geo.assign(s->tris.size() + kGeoPad, TriGeo{});
-  for (size_t i = 0; i < s->tris.size(); ++i) {
+  const int n = (int)s->tris.size();
+  std::vector<Prim> prims(n);
+  Box scene;
+  scene.clear();
+  for (int i = 0; i < n; ++i) {
+    const Tri& t = s->tris[i];
+    Prim& p = prims[i];
+    p.tri = i;
+    for (int k = 0; k < 3; ++k) {
+      const double a = comp(t.v0, k), b = comp(t.v1, k), c = comp(t.v2, k);
+      p.lo[k] = round_down_f(std::min(a, std::min(b, c)));
+      p.hi[k] = round_up_f(std::max(a, std::max(b, c)));
+      p.c[k] = p.lo[k] + p.hi[k];
+    }
+    scene.add(p.lo, p.hi);
+  }
+  float span = 0.0f, mag = 0.0f;
+  for (int k = 0; k < 3; ++k) {
+    span = std::max(span, scene.hi[k] - scene.lo[k]);
+    mag = std::max(mag, std::max(std::fabs(scene.lo[k]), std::fabs(scene.hi[k])));
+  }
+  const float margin = mag * kBoxMargin;
+  for (int k = 0; k < 3; ++k) {
+    s->lo[k] = round_down_f((double)scene.lo[k] - margin);
+    s->hi[k] = round_up_f((double)scene.hi[k] + margin);
+  }
+  std::vector<Node> bin;
+  for (int levels = 0; levels < 2; ++levels) {
+    build_binary(prims, span, levels ? 0 : 64, bin);
+    s->nodes.clear();
+    if (collapse8(s, bin, 0, margin, levels != 0) < kTraceStack) break;
+  }
+  s->order.resize(n);
+  s->geo.assign(n + kGeoPad, TriGeo{});
+  for (int i = 0; i < n; ++i) {
+    s->order[i] = prims[i].tri;
     const Tri& t = s->tris[s->order[i]];
     s->geo[i] = TriGeo{t.v0, t.v1 - t.v0, t.v2 - t.v0};
   }
@@ -536,7 +571,7 @@ int mlgi_scene_render_gbuffer(const mlgi_scene* s, const mlgi_camera* cam, int32
   const RayCam rc = ray_cam(cam);
   const SceneView sv = view_of(s);
   parallel_rows(h, nthreads(threads), [&](int y) {
-    StackTracer<LocalStack> tr;
+    StackTracer tr;
     for (int x = 0; x < w; ++x) shade_gbuffer(tr, sv, rc, x, y, w, h, depth, normal);
   });
   return MLGI_OK;
@@ -550,7 +585,7 @@ int mlgi_scene_render_rsm(const mlgi_scene* s, const mlgi_camera* light, int32_t
   const RayCam rc = ray_cam(light);
   const SceneView sv = view_of(s);
   parallel_rows(h, nthreads(threads), [&](int y) {
-    StackTracer<LocalStack> tr;
+    StackTracer tr;
     for (int x = 0; x < w; ++x) shade_rsm(tr, sv, rc, x, y, w, h, diffuse, normal, depth);
   });
   if (inv_bvp16 && !mlgi_scene_inv_biased_vp(light, inv_bvp16)) return MLGI_ERR_INVALID_ARGUMENT;
@@ -563,7 +598,7 @@ int mlgi_scene_render_surface(const mlgi_scene* s, const mlgi_camera* cam, int32
   const RayCam rc = ray_cam(cam);
   const SceneView sv = view_of(s);
   parallel_rows(h, nthreads(threads), [&](int y) {
-    StackTracer<LocalStack> tr;
+    StackTracer tr;
     for (int x = 0; x < w; ++x) shade_surface(tr, sv, rc, x, y, w, h, albedo, moments);
   });
   return MLGI_OK;
@@ -626,8 +661,8 @@ extern "C" int mlgi_scene_sample_points(const mlgi_scene* s, int64_t n_points, i
 
 namespace {
 SceneView view_of(const mlgi_scene* s) {
-  return SceneView{s->nodes4.data(), s->geo.data(), s->tris.data(), s->order.data(), (int)s->nodes4.size(),
-                   (int)s->tris.size()};
+  return SceneView{s->nodes.data(), s->geo.data(), s->tris.data(), s->order.data(), (int)s->nodes.size(),
+                   (int)s->tris.size(), {s->lo[0], s->lo[1], s->lo[2]}, {s->hi[0], s->hi[1], s->hi[2]}};
 }
 }  // namespace
 

@@ -35,30 +35,47 @@ struct Tri {
   float albedo[3];
 };
 
-// Binary BVH node of the build (scene.cpp); the ray caster walks the 4-wide
+// Binary BVH node of the build (scene.cpp); the ray casters walk the 8-wide
 // form below.
 struct Node {
-  double lo[3], hi[3];
-  // leaf: count > 0, left = first index; inner: left child (the smaller
-  // centroids along the split axis), right = left + 1, count = -1 - axis
+  float lo[3], hi[3];
+  // leaf: count > 0, left = first index; inner: left child, right = left + 1, count = 0
   int left, count;
 };
 
-// 4-wide BVH node: the binary tree with every inner node's grandchildren
-// pulled up into its child slots, stored as structures of arrays (the four
-// boxes and references of one node are one 128-byte line). Boxes are floats
-// rounded outward, so each still contains its triangles.
-struct alignas(16) Node4 {
-  float lo[3][4], hi[3][4];
-  int ref[4];    // inner child: node index; leaf child: first triangle (leaf order)
-  int count[4];  // leaf child: triangles (1..4); inner child: 0; empty slot: -1
+// 8-wide BVH node: eight child records of 32 bytes, the used ones first. The
+// boxes are floats that contain their triangles with a margin (kBoxMargin),
+// so that a slab test in FP32 keeps every box the exact ray touches.
+struct Child8 {
+  float lo[3], hi[3];
+  uint32_t ref;  // index << 3 | count: inner child: node index, count 0; leaf child: first triangle
+                 // (leaf order), 1..4 triangles; unused: kNoChild, with a box that no ray hits
+  // The children's front-to-back order per direction octant, in the eight
+  // children's words: octant o (bit a set: the ray runs towards smaller
+  // coordinates along axis a) < 4 takes words 2 o (children 0..3) and 2 o + 1
+  // (4..7); byte k is the set of children that come after child k. Octant
+  // o ^ 7 is the exact reverse.
+  uint32_t after;
 };
+struct alignas(16) Node8 {
+  Child8 c[8];
+};
+constexpr uint32_t kNoChild = 0xFFFFFFFFu;
+
+// Margin of the node boxes, as a share of the scene's largest coordinate
+// magnitude m. A ray's FP32 slab distances are off by at most (2^-21 + 2^-22) m
+// in position along an axis: the reciprocal direction (rounded direction and
+// hardware reciprocal, 2^-22 of a distance of at most 2 m), the rounded origin
+// (2^-24 m, the origin moved into the scene's box first), its product with the
+// reciprocal (2^-24 m) and the final sum (2^-24 of 2 m).
+constexpr float kBoxMargin = 0x1p-20f;
 
 // Triangle geometry in leaf order for the intersection test: v0 and the two
 // edges v1 - v0, v2 - v0 (computed once, in double, as the test would). The
 // array carries three zero entries past the last triangle, so that a leaf's
 // four slots can be loaded without a bounds test.
 constexpr int kGeoPad = 3;
+constexpr int kLeafTris = 4;
 struct TriGeo {
   D3 v0, e1, e2;
 };
@@ -70,16 +87,16 @@ struct Hit {
 
 // The scene as flat arrays (host vectors or device copies).
 struct SceneView {
-  const Node4* nodes4;
-  const TriGeo* geo;  // leaf order
-  const Tri* tris;    // scene order (normals, albedo, sampling)
-  const int* order;   // leaf order -> scene order
-  int n_nodes4, n_tris;
+  const Node8* nodes;  // nodes[0] is the root
+  const TriGeo* geo;   // leaf order
+  const Tri* tris;     // scene order (normals, albedo, sampling)
+  const int* order;    // leaf order -> scene order
+  int n_nodes, n_tris;
+  float lo[3], hi[3];  // the scene's box, with the nodes' margin
 };
 
-// Slab test of a float box (bounds taken exactly into double), without early
-// exits: t0 only grows and t1 only shrinks, so testing once after the three
-// axes gives the same answer.
+// Slab test of a float box in double, without early exits: t0 only grows and
+// t1 only shrinks, so testing once after the three axes gives the same answer.
 MLGI_HD inline bool box_hit(const float lo_[3], const float hi_[3], D3 o, D3 inv, double tmax, double* tnear) {
   double t0 = 0.0, t1 = tmax;
   for (int k = 0; k < 3; ++k) {
@@ -93,168 +110,112 @@ MLGI_HD inline bool box_hit(const float lo_[3], const float hi_[3], D3 o, D3 inv
   return !(t0 > t1);
 }
 
-// Child slot c of a 4-wide node.
-MLGI_HD inline bool box4_hit(const Node4& nd, int c, D3 o, D3 inv, double tmax, double* tnear) {
-  const float lo[3] = {nd.lo[0][c], nd.lo[1][c], nd.lo[2][c]};
-  const float hi[3] = {nd.hi[0][c], nd.hi[1][c], nd.hi[2][c]};
-  return box_hit(lo, hi, o, inv, tmax, tnear);
+// Moller-Trumbore, two-sided, in two steps: the determinant and the three
+// numerators, then, where tri_maybe has not ruled the triangle out by signs
+// and magnitudes alone (no division), the quotients and the exact tests.
+struct TriTerms {
+  double det, u, v, t;
+};
+MLGI_HD inline TriTerms tri_terms(const TriGeo& g, D3 o, D3 d) {
+  const D3 p = cross(d, g.e2);
+  const D3 s = o - g.v0;
+  const D3 q = cross(s, g.e1);
+  return TriTerms{dot(g.e1, p), dot(s, p), dot(d, q), dot(g.e2, q)};
 }
-
-// Moller-Trumbore, two-sided
-MLGI_HD inline bool tri_hit(const TriGeo& g, D3 o, D3 d, double tmax, double* th) {
-  D3 p = cross(d, g.e2);
-  double det = dot(g.e1, p);
-  if (fabs(det) < 1e-14) return false;
-  double inv = 1.0 / det;
-  D3 s = o - g.v0;
-  double u = dot(s, p) * inv;
+// False only where tri_accept is false: a quotient has the sign of its
+// numerator times the determinant's, and one over 1 + 1e-10 (or over
+// tmax (1 + 1e-10)) stays over its limit after any rounding.
+MLGI_HD inline bool tri_maybe(const TriTerms& k, double tmax) {
+  const double a = fabs(k.det);
+  const double u = k.det < 0.0 ? -k.u : k.u, v = k.det < 0.0 ? -k.v : k.v, t = k.det < 0.0 ? -k.t : k.t;
+  const double lim = a * (1.0 + 1e-10);
+  return (a >= 1e-14) & (u >= 0.0) & (v >= 0.0) & (u + v <= lim) & (t > 0.0) & (t <= lim * tmax);
+}
+// The exact test of a triangle that tri_maybe let through: t in (0, tmax].
+MLGI_HD inline bool tri_accept(const TriTerms& k, double tmax, double* th) {
+  const double inv = 1.0 / k.det;
+  const double u = k.u * inv;
   if (u < 0.0 || u > 1.0) return false;
-  D3 q = cross(s, g.e1);
-  double v = dot(d, q) * inv;
+  const double v = k.v * inv;
   if (v < 0.0 || u + v > 1.0) return false;
-  double tt = dot(g.e2, q) * inv;
-  if (tt <= 0.0 || tt >= tmax) return false;
+  const double tt = k.t * inv;
+  if (tt <= 0.0 || tt > tmax) return false;
   *th = tt;
   return true;
 }
+// Whether a hit of triangle i (leaf order) at t replaces h: the nearer one, of
+// equally near ones the first in leaf order, whatever order they were found
+// in. A hit at the ray's end is none.
+MLGI_HD inline bool hit_before(double t, int i, const Hit& h) { return t < h.t || (t == h.t && i < h.tri); }
 
-// Pending children of the traversal: at most three per level of the 4-wide
-// tree, whose depth the build keeps within 16 (binary depth 32).
-constexpr int kTraceStack = 48;
+// Pending children of a traversal; the build keeps every path's sum of
+// (children - 1) below it.
+constexpr int kTraceStack = 128;
 
-// A pending child: ref << 3 | count (inner node: count 0; leaf: 1..4
-// triangles) and its box's entry distance rounded down to a float (the pop
-// test then never drops a box the exact test would keep).
+// A pending child and its box's entry distance.
 struct StackEntry {
-  int rc;
-  float tnear;
+  uint32_t ref;
+  double tnear;
 };
-
-// Traversal stack in the caller's memory (host: a local array).
 struct LocalStack {
   StackEntry e[kTraceStack];
-  MLGI_HD void put(int i, const StackEntry& v) { e[i] = v; }
-  MLGI_HD StackEntry get(int i) const { return e[i]; }
 };
 
-// Largest float <= x for x >= 0 (a rounded-up f is then > 0: one step down
-// is the previous float).
-MLGI_HD inline float round_down_f(double x) {
-  float f = (float)x;
-  if ((double)f > x) {
-    union {
-      float f;
-      uint32_t u;
-    } b;
-    b.f = f;
-    b.u -= 1u;
-    f = b.f;
-  }
-  return f;
-}
-
-// Compare-exchange of the child order: by entry distance, then slot.
-MLGI_HD inline void order2(double* t, int* slot, int* rc, int i, int j) {
-  if (t[i] > t[j] || (t[i] == t[j] && slot[i] > slot[j])) {
-    const double tt = t[i];
-    t[i] = t[j];
-    t[j] = tt;
-    const int ss = slot[i];
-    slot[i] = slot[j];
-    slot[j] = ss;
-    const int rr = rc[i];
-    rc[i] = rc[j];
-    rc[j] = rr;
-  }
-}
-
-// Nearest hit with t < tmax. At an inner node the whole 128-byte node is read
-// at once and its four child boxes tested, the hit children are ordered by
-// entry distance (then slot; missed slots last), the nearest is visited and
-// the others pushed, farthest first. A popped child is skipped if its box is
-// entered beyond the current nearest hit. Leaves test their triangles in leaf
-// order; among hits at exactly equal t the first one reached wins. All array
-// indices are compile-time (registers, no private memory), and host and
-// device run this same code, so they take the same decisions.
+// Nearest hit with t < tmax, on the host: an inner node's child boxes are
+// tested, the hit ones pushed, farthest first; a popped child is skipped if
+// its box is entered beyond the nearest hit so far. The device walks the same
+// nodes in packets (raycast.hip). Which of the triangles is nearest, and which
+// of equally near ones wins, does not depend on the order of the visits, so
+// both give the same hit.
 MLGI_HD inline D3 ray_inverse(D3 d) {
   return {1.0 / (d.x != 0 ? d.x : 1e-300), 1.0 / (d.y != 0 ? d.y : 1e-300), 1.0 / (d.z != 0 ? d.z : 1e-300)};
 }
 
-// Entry distance of a missed child slot: orders after every hit one.
-constexpr double kMissed = 1e300;
-
-// The ordering network of an inner step: hit children by entry distance,
-// then slot; missed slots last.
-MLGI_HD inline void order_children(double* tk, int* slot, int* rc) {
-  order2(tk, slot, rc, 0, 1);
-  order2(tk, slot, rc, 2, 3);
-  order2(tk, slot, rc, 0, 2);
-  order2(tk, slot, rc, 1, 3);
-  order2(tk, slot, rc, 1, 2);
-}
-
-template <class Stack>
-MLGI_HD inline Hit trace(const SceneView& s, D3 o, D3 d, double tmax, Stack& st) {
+inline Hit trace(const SceneView& s, D3 o, D3 d, double tmax, LocalStack& st) {
   Hit h{tmax, -1};
   const D3 inv = ray_inverse(d);
   int sp = 0;
-  int ref = 0, count = 0;  // the root, an inner node
+  uint32_t cur = 0;  // the root, an inner node
   while (true) {
+    const int count = (int)(cur & 7u), first = (int)(cur >> 3);
     if (count == 0) {
-      const Node4 nd = s.nodes4[ref];
-      double tk[4];
-      int slot[4], rc[4];
-      for (int k = 0; k < 4; ++k) {
+      const Node8& nd = s.nodes[first];
+      const int base = sp;
+      for (int k = 0; k < 8 && nd.c[k].ref != kNoChild; ++k) {
         double tn;
-        const bool hit = box4_hit(nd, k, o, inv, h.t, &tn) && nd.count[k] >= 0;
-        tk[k] = hit ? tn : kMissed;
-        slot[k] = k;
-        rc[k] = (nd.ref[k] << 3) | (nd.count[k] & 7);
-      }
-      order_children(tk, slot, rc);
-      for (int i = 3; i >= 1; --i)  // never full (see kTraceStack); checked all the same
-        if (tk[i] < kMissed && sp < kTraceStack) st.put(sp++, StackEntry{rc[i], round_down_f(tk[i])});
-      if (tk[0] < kMissed) {
-        ref = rc[0] >> 3;
-        count = rc[0] & 7;
-        continue;
+        if (!box_hit(nd.c[k].lo, nd.c[k].hi, o, inv, h.t, &tn)) continue;
+        int i = sp++;  // insert, the nearest last (never full: see kTraceStack)
+        for (; i > base && st.e[i - 1].tnear < tn; --i) st.e[i] = st.e[i - 1];
+        st.e[i] = StackEntry{nd.c[k].ref, tn};
       }
     } else {
-      TriGeo g[4];
-      for (int k = 0; k < 4; ++k) g[k] = s.geo[ref + k];  // padded: in bounds for every leaf
-      for (int k = 0; k < 4; ++k) {
+      for (int k = 0; k < count; ++k) {
+        const TriTerms q = tri_terms(s.geo[first + k], o, d);
         double th;
-        if (k < count && tri_hit(g[k], o, d, h.t, &th)) {
+        if (tri_maybe(q, h.t) && tri_accept(q, h.t, &th) && hit_before(th, first + k, h)) {
           h.t = th;
-          h.tri = ref + k;
+          h.tri = first + k;
         }
       }
     }
-    bool more = false;
-    while (sp > 0) {
-      const StackEntry e = st.get(--sp);
-      if (!((double)e.tnear > h.t)) {
-        ref = e.rc >> 3;
-        count = e.rc & 7;
-        more = true;
-        break;
+    do {
+      if (sp == 0) {
+        if (h.tri >= 0) h.tri = s.order[h.tri];
+        return h;
       }
-    }
-    if (!more) break;
+      --sp;
+    } while (st.e[sp].tnear > h.t);
+    cur = st.e[sp].ref;
   }
-  if (h.tri >= 0) h.tri = s.order[h.tri];
-  return h;
 }
 
-// One ray per thread over a traversal stack (the host renderer; the device's
-// one-lane-per-texel form). The shading functions below call a tracer and
-// store only where it says so (a cooperative device tracer has several lanes
-// per ray, one of which stores).
-template <class Stack>
+// One ray per call (the host renderer). The shading functions below call a
+// tracer and store only where it says so (the device's packet tracers run
+// whole waves, some lanes of which do not store).
 struct StackTracer {
-  Stack st;
-  MLGI_HD Hit operator()(const SceneView& s, D3 o, D3 d, double tmax) { return trace(s, o, d, tmax, st); }
-  MLGI_HD bool stores() const { return true; }
+  LocalStack st;
+  Hit operator()(const SceneView& s, D3 o, D3 d, double tmax) { return trace(s, o, d, tmax, st); }
+  bool stores() const { return true; }
 };
 
 // 4x4 column-major, double
