@@ -29,8 +29,8 @@
 //     atomic umin. If the list overflowed, it instead reruns the point-major
 //     splat of the whole frame over the tiles; min is idempotent, so the
 //     result is the same.
-// Tiles are mapped to XCDs in contiguous ranges, so the bins that
-// neighbouring ISMs share are read through one L2.
+// Bins and ISMs are dealt to the XCDs in chunks of 32 neighbours (xcd_item),
+// so the bins that neighbouring ISMs share are mostly read through one L2.
 #include <algorithm>
 #include <mutex>
 
@@ -485,9 +485,9 @@ __device__ __forceinline__ TileJob tile_job(const BatchFrame& f) {
                  f.ism_side, f.atlas_side, f.z_far, f.atlas, f.mask, f.spill_state, f.spill};
 }
 
-// Single-frame kernels: one workgroup per item (xcd_item), XCD x taking one
-// contiguous eighth of the items (a persistent grid walking them measured
-// slower: the hardware balances retiring workgroups better).
+// Single-frame kernels: one workgroup per item (xcd_item; a persistent grid
+// walking them measured slower: the hardware balances retiring workgroups
+// better).
 __global__ __launch_bounds__(256) void ism_mask_kernel(TileJob j, int n_bins) {
   __shared__ Candidate cand[kMaxTest];
   const uint32_t b = xcd_item((uint32_t)n_bins);
