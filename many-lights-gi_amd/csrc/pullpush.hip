@@ -653,8 +653,11 @@ __device__ __forceinline__ void list_append2(uint16_t* list, int* count, bool ta
   if (take1) list[first + n0 + lanes_below(m1)] = (uint16_t)v1;
 }
 
+// The pull levels from l on. False when the group's tiles hold no sample at
+// all, which the two-pass first level finds out: nothing above it is built
+// then (empty_tiles).
 template <int S, int l, int L>
-__device__ __forceinline__ void pull_levels(const Tables& tb, const PullConsts& pc) {
+__device__ __forceinline__ bool pull_levels(const Tables& tb, const PullConsts& pc) {
   if constexpr (l <= L) {
     constexpr int so = S >> l, n = so * so;
     const int total = group_count<S>(tb.groups) * n;
@@ -686,12 +689,30 @@ __device__ __forceinline__ void pull_levels(const Tables& tb, const PullConsts& 
       }
       __syncthreads();
       const int count = tb.counts[0];
+      if (count == 0) return false;
       for (int i = threadIdx.x; i < count; i += kThreads) full(list[i]);
     } else {
       for (int t = threadIdx.x; t < total; t += kThreads) full(t);
     }
     __syncthreads();
-    pull_levels<S, l + 1, L>(tb, pc);
+    return pull_levels<S, l + 1, L>(tb, pc);
+  }
+  return true;
+}
+
+// The result of a group without a sample (the ISMs past the VPL count in a
+// grid they do not fill: half of a 2,048-VPL frame's). Every depth its pull
+// and push levels could hold is 1 - 2^-24 or a rounded weighted mean of such
+// depths, within 2^-21 of 1, and anything within 2^-17 of 1 is 65535.
+template <int S>
+__device__ __forceinline__ void empty_tiles(const Tables& tb) {
+  constexpr int kRow = S / 4, n = S * kRow;  // 8-byte stores, four texels each
+  typedef unsigned int v2u __attribute__((ext_vector_type(2)));
+  const v2u ones = {0xFFFFFFFFu, 0xFFFFFFFFu};
+  for (int t = threadIdx.x; t < group_count<S>(tb.groups) * n; t += kThreads) {
+    const int g = t / n, o = t - g * n;
+    const uint32_t at = tb.origin(S, g) + ((uint32_t)(o / kRow) << tb.side_log2) + 4u * (uint32_t)(o % kRow);
+    __builtin_amdgcn_raw_buffer_store_b64(ones, tb.out, at * 2u, 0, 0);
   }
 }
 
@@ -762,7 +783,10 @@ __device__ __forceinline__ void pullpush_tile(TileLds<S, L>& sm, const uint32_t*
   const float r255 = (float)255 / 10.0f;
   tb.empty = decode_texel(0xFFFFFFFFu, r255, r255 * 2.0f / z_far * 0.6f, z_far, S);
 
-  pull_levels<S, 1, L>(tb, pc);
+  if (!pull_levels<S, 1, L>(tb, pc)) {
+    empty_tiles<S>(tb);
+    return;
+  }
   if constexpr (L == 1) {
     // no level-1 push stores the bounds the level-0 push reads
     constexpr int n1 = (S / 2) * (S / 2);
