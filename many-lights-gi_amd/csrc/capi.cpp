@@ -1376,21 +1376,19 @@ int mlgi_scene_device_sample_points(mlgi_context* c, const mlgi_scene_device* d,
                 n_bins, ism_count);
   const int n = (int)n_points;
   const float r_packed = mlgi_scene_point_radius(d->total_area, n_points, ism_count);
-  float* tmp = nullptr;
-  int* bin = nullptr;
-  uint32_t* cnt = nullptr;
-  int rc = hip_check(c, hipMalloc(&tmp, sizeof(float) * 4 * (size_t)std::max(n, 1)), "hipMalloc(points tmp)");
-  if (!rc) rc = hip_check(c, hipMalloc(&bin, sizeof(int) * (size_t)std::max(n, 1)), "hipMalloc(points bin)");
-  if (!rc) rc = hip_check(c, hipMalloc(&cnt, sizeof(uint32_t) * 2 * (size_t)n_bins), "hipMalloc(points count)");
+  // one work area: records, places, counts
+  const size_t rec_bytes = sizeof(float) * 4 * (size_t)n, place_bytes = sizeof(uint2) * (size_t)n;
+  char* work = nullptr;
+  int rc = hip_check(c, hipMalloc(&work, rec_bytes + place_bytes + sizeof(uint32_t) * (size_t)n_bins),
+                     "hipMalloc(points work)");
   if (!rc)
     rc = hip_check(c,
                    mlgi::launch_sample_points(c->stream, d->tris, d->cdf, d->n_tris, d->total_area, seed, r_packed,
-                                              n_bins, n, tmp, bin, cnt, cnt + n_bins, records, bin_offsets),
+                                              n_bins, n, (float*)work, (uint2*)(work + rec_bytes),
+                                              (uint32_t*)(work + rec_bytes + place_bytes), records, bin_offsets),
                    "sample_points");
   if (!rc) rc = hip_check(c, hipStreamSynchronize(c->stream), "hipStreamSynchronize");
-  if (tmp) (void)hipFree(tmp);
-  if (bin) (void)hipFree(bin);
-  if (cnt) (void)hipFree(cnt);
+  if (work) (void)hipFree(work);
   return rc;
 }
 

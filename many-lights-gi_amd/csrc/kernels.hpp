@@ -137,10 +137,10 @@ struct Tri;
 }  // namespace mlgi_scene_impl
 namespace mlgi {
 // points.hip: device point set of a scene (records grouped by bin). Work
-// buffers: tmp (4n floats), bin (n), count and cursor (n_bins each).
+// buffers: tmp (4n floats), place (n: bin, place in the bin), count (n_bins).
 hipError_t launch_sample_points(hipStream_t s, const mlgi_scene_impl::Tri* tris, const double* cdf, int nt,
-                                double total, uint64_t seed, float r_packed, int n_bins, int n, float* tmp, int* bin,
-                                uint32_t* count, uint32_t* cursor, float* records, uint32_t* offsets);
+                                double total, uint64_t seed, float r_packed, int n_bins, int n, float* tmp,
+                                uint2* place, uint32_t* count, float* records, uint32_t* offsets);
 hipError_t launch_raycast(hipStream_t st, const mlgi_scene_impl::SceneView& s,
                           const mlgi_scene_impl::RayCam& rc, int w, int h, int rsm, float* a, float* b,
                           float* c);
