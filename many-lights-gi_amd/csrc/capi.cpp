@@ -1044,6 +1044,10 @@ int batch_plan(mlgi_context* c, const mlgi_frame_desc* frames, int count, std::v
   plan->row_of.assign(count, 0);
   for (int r = 0; r < count; ++r) plan->row_of[order[r]] = r;
   table->assign(count, mlgi::BatchFrame{});
+  std::map<int, uint64_t> isms;  // of each pull-push launch
+  for (int i = 0; i < count; ++i) isms[key[i]] += (uint64_t)rows[i].n1d * rows[i].n1d;
+  for (int i = 0; i < count; ++i)
+    rows[i].pp_group = mlgi::pullpush_group(rows[i].ism_side, isms[key[i]], rows[i].n1d * rows[i].n1d);
   uint64_t tv = 0, tt = 0, tb = 0;
   size_t work = 0;
   for (int r = 0; r < count; ++r) {
@@ -1132,7 +1136,7 @@ mlgi::BatchCounts mlgi::batch_counts(const mlgi::BatchFrame& f) {
   n.vpl = (uint32_t)f.g.n_vpl;
   n.tiles = (uint32_t)(f.n1d * f.n1d);
   n.bins = f.n_points > 0 ? (uint32_t)f.g.n_vpl : 0u;
-  n.pp = (uint32_t)(f.n1d * f.n1d / mlgi::pullpush_group(f.ism_side, f.n1d * f.n1d));
+  n.pp = (uint32_t)(f.n1d * f.n1d / f.pp_group);
   const int th = 64 >> f.wave_w_log2;
   const int ch = (f.g.height + f.g.interleave - 1) / f.g.interleave;
   const uint32_t strips_y = (uint32_t)((ch + th - 1) / th);

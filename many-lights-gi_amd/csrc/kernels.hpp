@@ -169,6 +169,7 @@ struct BatchFrame {
   uint32_t* spill_state;
   uint2* spill;
   int atlas_side, ism_side, n1d, levels;
+  int pp_group;  // ISMs per pull-push workgroup (pullpush_group)
   float z_far;
   uint32_t pp_e1[4];  // pull level 1 of an all-empty block (bits of depth, maxDepth, radius, disp)
   // final gather (g.vpl = VPL records, g.ism = unorm16 ISM atlas, g.out)
@@ -184,11 +185,17 @@ struct BatchCounts {
   uint32_t vpl, tiles, bins, pp, waves;  // pp: pull-push items (ISM groups, pullpush_group)
 };
 
-// ISMs of side S that one pull-push workgroup takes: as many as make 64^2
-// texels, at most the frame's n_isms (both powers of four, so it divides).
-__host__ __device__ inline int pullpush_group(int ism_side, int n_isms) {
-  const int g = (64 / ism_side) * (64 / ism_side);
-  return g < n_isms ? g : n_isms;
+// ISMs of side S that one pull-push workgroup takes, of the launch's total
+// (all ISMs of the frames with this side and level count): as many as make
+// 64^2 texels, so that the small levels of several ISMs share wave iterations,
+// but fewer where that leaves under 512 workgroups: a launch that does not
+// fill the chip (256 CUs) is bound by one workgroup's latency, which falls
+// with its share. A power of four at most `total`, as every frame's ISM count
+// is, so it divides each.
+inline int pullpush_group(int ism_side, uint64_t total, int n_isms) {
+  int g = (64 / ism_side) * (64 / ism_side);
+  while (g > 1 && (g > n_isms || total / (uint64_t)g < 512)) g /= 4;
+  return g;
 }
 BatchCounts batch_counts(const BatchFrame& f);
 

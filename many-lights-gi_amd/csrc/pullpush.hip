@@ -822,7 +822,7 @@ __global__ __launch_bounds__(kThreads) void batch_pullpush_kernel(const BatchFra
   PullConsts pc;
   pc.e1 = Texel{__uint_as_float(f.pp_e1[0]), __uint_as_float(f.pp_e1[1]), __uint_as_float(f.pp_e1[2]),
                 f.pp_e1[3]};
-  const int groups = pullpush_group(S, f.n1d * f.n1d);
+  const int groups = f.pp_group;
   pullpush_tile<S, L>(sm, f.atlas, f.atlas_side, f.z_far, pc, const_cast<uint16_t*>(f.g.ism),
                       (int)(item - f.first_pp) * groups, groups);
 }
@@ -852,7 +852,7 @@ template <int S, int L>
 hipError_t launch_sl(hipStream_t s, const uint32_t* atlas, int atlas_side, float z_far,
                      const PullConsts& pc, uint16_t* out) {
   const int n1d = atlas_side / S;
-  const int groups = pullpush_group(S, n1d * n1d);
+  const int groups = pullpush_group(S, (uint64_t)n1d * n1d, n1d * n1d);
   hipLaunchKernelGGL((pullpush_kernel<S, L>), dim3(n1d * n1d / groups), dim3(kThreads), 0, s, atlas, atlas_side,
                      z_far, pc, out, groups);
   return hipGetLastError();
