@@ -1438,3 +1438,19 @@ int mlgi_scene_device_render_rsm(mlgi_context* c, const mlgi_scene_device* d, co
 }
 
 }  // extern "C"
+
+int mlgi_capi::rsm_job(mlgi_context* c, const mlgi_scene_device* d, const mlgi_camera* light, int w, int h,
+                       float* diffuse, float* normal, float* depth, float inv_bvp16[16],
+                       mlgi_scene_impl::RsmJob* out) {
+  if (!d || !light || !diffuse || !normal || !depth) return fail(c, MLGI_ERR_INVALID_ARGUMENT, "NULL argument");
+  if (w <= 0 || h <= 0 || w > 16384 || h > 16384)
+    return fail(c, MLGI_ERR_INVALID_ARGUMENT, "size %dx%d out of range", w, h);
+  out->scene = d->view();
+  out->diffuse = diffuse;
+  out->normal = normal;
+  out->depth = depth;
+  if (!mlgi_scene_ray_cam(light, &out->light)) return fail(c, MLGI_ERR_INVALID_ARGUMENT, "bad light");
+  if (inv_bvp16 && !mlgi_scene_inv_biased_vp(light, inv_bvp16))
+    return fail(c, MLGI_ERR_INVALID_ARGUMENT, "singular light");
+  return MLGI_OK;
+}

@@ -125,6 +125,10 @@ int batch_plan(mlgi_context* c, const mlgi_frame_desc* frames, int count, std::v
 // Points the table rows' splat work areas into `base` (plan.work_bytes bytes
 // of device memory, one area per frame).
 void batch_attach_work(std::vector<mlgi::BatchFrame>* table, char* base);
+// The render of a light's RSM (w x h texels) as a job of launch_rsms; also its
+// inverse biased light matrix.
+int rsm_job(mlgi_context* c, const mlgi_scene_device* d, const mlgi_camera* light, int w, int h, float* diffuse,
+            float* normal, float* depth, float inv_bvp16[16], mlgi_scene_impl::RsmJob* out);
 // Enqueues a planned batch whose table is at `dev` (device memory).
 int batch_enqueue(mlgi_context* c, const mlgi::BatchFrame* dev, const BatchPlan& plan);
 

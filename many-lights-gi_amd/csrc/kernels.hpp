@@ -133,6 +133,7 @@ hipError_t launch_division_check(hipStream_t s, uint32_t* counts, uint32_t seed)
 namespace mlgi_scene_impl {
 struct SceneView;
 struct RayCam;
+struct RsmJob;
 struct Tri;
 }  // namespace mlgi_scene_impl
 namespace mlgi {
@@ -141,6 +142,9 @@ namespace mlgi {
 hipError_t launch_sample_points(hipStream_t s, const mlgi_scene_impl::Tri* tris, const double* cdf, int nt,
                                 double total, uint64_t seed, float r_packed, int n_bins, int n, float* tmp,
                                 uint2* place, uint32_t* count, float* records, uint32_t* offsets);
+// n RSMs of w x h texels, up to kRsmJobs of them in one launch: one 128^2 RSM
+// is a wave per SIMD bound by its longest packet, and others fit beside it.
+hipError_t launch_rsms(hipStream_t st, const mlgi_scene_impl::RsmJob* jobs, int n, int w, int h);
 hipError_t launch_raycast(hipStream_t st, const mlgi_scene_impl::SceneView& s,
                           const mlgi_scene_impl::RayCam& rc, int w, int h, int rsm, float* a, float* b,
                           float* c);

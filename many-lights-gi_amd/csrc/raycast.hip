@@ -368,7 +368,46 @@ __global__ __launch_bounds__(64) void raycast_quad_kernel(SceneView s, RayCam rc
   shade(tr, s, rc, min(x, w - 1), min(y, h - 1), w, h, mode, a, b, c);
 }
 
+struct RsmJobs {
+  RsmJob j[kRsmJobs];
+};
+static_assert(sizeof(RsmJobs) + 2 * sizeof(int) <= 4096, "kernel arguments");
+
+// The RSM of job blockIdx.z, as the two kernels above.
+__global__ __launch_bounds__(64) void rsms_kernel(RsmJobs jobs, int w, int h) {
+  __shared__ PacketLds<64> lds;
+  const RsmJob& job = jobs.j[blockIdx.z];
+  const int x = blockIdx.x * 8 + (threadIdx.x & 7);
+  const int y = blockIdx.y * 8 + (threadIdx.x >> 3);
+  RayTracer tr{lds, x < w && y < h};
+  shade_rsm(tr, job.scene, job.light, min(x, w - 1), min(y, h - 1), w, h, job.diffuse, job.normal, job.depth);
+}
+__global__ __launch_bounds__(64) void rsms_quad_kernel(RsmJobs jobs, int w, int h) {
+  __shared__ PacketLds<16> lds;
+  const RsmJob& job = jobs.j[blockIdx.z];
+  const int q = threadIdx.x & 3, r = threadIdx.x >> 2;
+  const int x = blockIdx.x * 4 + (r & 3);
+  const int y = blockIdx.y * 4 + (r >> 2);
+  QuadTracer tr{lds, q == 0 && x < w && y < h};
+  shade_rsm(tr, job.scene, job.light, min(x, w - 1), min(y, h - 1), w, h, job.diffuse, job.normal, job.depth);
+}
+
 }  // namespace
+
+hipError_t launch_rsms(hipStream_t st, const RsmJob* jobs, int n, int w, int h) {
+  for (int i = 0; i < n; i += kRsmJobs) {
+    const int m = n - i < kRsmJobs ? n - i : kRsmJobs;
+    RsmJobs group = {};
+    for (int k = 0; k < m; ++k) group.j[k] = jobs[i + k];
+    if ((size_t)w * (size_t)h * (size_t)m <= kWideRays)
+      hipLaunchKernelGGL(rsms_quad_kernel, dim3((w + 3) / 4, (h + 3) / 4, m), dim3(64), 0, st, group, w, h);
+    else
+      hipLaunchKernelGGL(rsms_kernel, dim3((w + 7) / 8, (h + 7) / 8, m), dim3(64), 0, st, group, w, h);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
+}
 
 hipError_t launch_raycast(hipStream_t st, const SceneView& s, const RayCam& rc, int w, int h, int rsm,
                           float* a, float* b, float* c) {

@@ -236,6 +236,14 @@ struct RayCam {
   double cos_half;  // spot cone (RSM only)
 };
 
+// One RSM render of a group (launch_rsms): scene, light, output planes.
+struct RsmJob {
+  SceneView scene;
+  RayCam light;
+  float *diffuse, *normal, *depth;
+};
+constexpr int kRsmJobs = 8;  // per launch: the jobs are kernel arguments (4 KiB)
+
 // Ray through the pixel centre from the near plane to the far plane.
 MLGI_HD inline void pixel_ray(const RayCam& rc, int x, int y, int w, int h, D3* o, D3* d) {
   double nx = ((x + 0.5) / w) * 2.0 - 1.0, ny = ((y + 0.5) / h) * 2.0 - 1.0;

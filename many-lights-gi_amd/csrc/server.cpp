@@ -37,6 +37,7 @@
 #include "../../include/mlgi_scene.h"
 #include "capi_internal.hpp"
 #include "kernels.hpp"
+#include "scene_trace.hpp"
 
 using namespace mlgi_capi;
 
@@ -230,9 +231,9 @@ mlgi_frame_desc request_frame(mlgi_server* s, const mlgi_request& r, size_t off,
   return d;
 }
 
-// Renders the request's RSM on lane L's stream (asynchronous) and returns its
-// inverse biased light matrix.
-int render_request_rsm(mlgi_server* s, mlgi_context* L, const mlgi_request& r, size_t off, float inv_bvp[16]) {
+// The render of the request's RSM, and its inverse biased light matrix.
+int request_rsm(mlgi_server* s, mlgi_context* L, const mlgi_request& r, size_t off, float inv_bvp[16],
+                mlgi_scene_impl::RsmJob* job) {
   const int rs = s->cfg.rsm_size;
   const Footprint fp = footprint(r.width, r.height, r.n_vpl, rs, points_of(s, r));
   char* b = s->arena_base + off;
@@ -241,7 +242,13 @@ int render_request_rsm(mlgi_server* s, mlgi_context* L, const mlgi_request& r, s
   float* dep = (float*)((char*)nrm + fp.rsm_normal);
   mlgi_camera light;
   mlgi_scene_light_pose(r.light_seed, &light);
-  return mlgi_scene_device_render_rsm(L, s->scenes[r.scene].dev, &light, rs, rs, dif, nrm, dep, inv_bvp);
+  return rsm_job(L, s->scenes[r.scene].dev, &light, rs, rs, dif, nrm, dep, inv_bvp, job);
+}
+
+// Renders RSMs on lane L's stream (asynchronous).
+int render_rsms(mlgi_server* s, mlgi_context* L, const std::vector<mlgi_scene_impl::RsmJob>& jobs) {
+  return hip_check(L, mlgi::launch_rsms(L->stream, jobs.data(), (int)jobs.size(), s->cfg.rsm_size, s->cfg.rsm_size),
+                   "raycast(rsm)");
 }
 
 // Copies a lane's error into the server context's (no-op for lane 0).
@@ -371,7 +378,8 @@ int mlgi_server_create(mlgi_context* c, const mlgi_server_config* cfg, const mlg
       size_t off = 0;
       s->arena.alloc(fp.total, &off);
       float inv[16];
-      if ((rc = render_request_rsm(s, c, r, off, inv))) break;
+      std::vector<mlgi_scene_impl::RsmJob> job(1);
+      if ((rc = request_rsm(s, c, r, off, inv, &job[0])) || (rc = render_rsms(s, c, job))) break;
       Tune t{4, 8, 8};
       mlgi_frame_desc d = request_frame(s, r, off, t, inv, nullptr);
       mlgi_tune_result tr;
@@ -446,6 +454,7 @@ int mlgi_server_run(mlgi_server* s, const mlgi_request* reqs, int32_t n, mlgi_se
       mlgi_context* L = s->lane_of(slot);
       std::vector<Admitted> adm;
       std::vector<mlgi_frame_desc> descs;
+      std::vector<mlgi_scene_impl::RsmJob> rsms;
       while (!queue.empty() && (int)adm.size() < s->cfg.max_batch && inflight_reqs < s->cfg.max_inflight) {
         const int i = queue.front();
         const mlgi_request& r = reqs[i];
@@ -461,12 +470,14 @@ int mlgi_server_run(mlgi_server* s, const mlgi_request* reqs, int32_t n, mlgi_se
         if (!s->arena.alloc(fp.total, &off)) break;  // wait for releases (FIFO, no overtaking)
         queue.pop_front();
         float inv[16];
-        if ((rc = lane_fail(s, L, render_request_rsm(s, L, r, off, inv)))) break;
+        rsms.emplace_back();
+        if ((rc = lane_fail(s, L, request_rsm(s, L, r, off, inv, &rsms.back())))) break;
         float* img = nullptr;
         descs.push_back(request_frame(s, r, off, s->tuned.at({r.width, r.height, r.n_vpl}), inv, &img));
         adm.push_back({i, off, fp.total, img});
         ++inflight_reqs;
       }
+      if (!rc && !adm.empty()) rc = lane_fail(s, L, render_rsms(s, L, rsms));
       if (!rc && !adm.empty()) {
         ring_free.pop_back();
         std::vector<mlgi::BatchFrame> table;
