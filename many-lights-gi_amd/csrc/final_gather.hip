@@ -247,7 +247,9 @@ struct LitConsts {
 // 64-bit address arithmetic of a global load per lit pair. Resource word 3
 // 0x00020000 selects the 32-bit data format raw buffer loads use on CDNA.
 __device__ __forceinline__ LitConsts lit_consts(const GatherArgs& a) {
-  return LitConsts{__builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(a.ism), 0, 0x7FFFFFFF, 0x00020000),
+  return LitConsts{__builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(a.ism), 0,
+                                                     (int)((uint32_t)a.atlas_side * (uint32_t)a.atlas_side * 2u),
+                                                     0x00020000),
                    0.5f * (float)a.ism_side, a.atlas_side - 1, 31 - __builtin_clz(a.atlas_side),
                    a.shadow_k1, a.shadow_k2};
 }
@@ -256,6 +258,13 @@ __device__ __forceinline__ LitConsts lit_consts(const GatherArgs& a) {
 // GL_REPEAT wraps the atlas.
 __device__ __forceinline__ uint32_t atlas_texel(const LitConsts& lc, int ox, int oy, int tx, int ty) {
   return (uint32_t)((((oy + ty) & lc.amask) << lc.alog) | ((ox + tx) & lc.amask));
+}
+
+// int(floor(x)), saturating, in one instruction.
+__device__ __forceinline__ int floor_int(float x) {
+  int r;
+  asm("v_cvt_flr_i32_f32 %0, %1" : "=v"(r) : "v"(x));
+  return r;
 }
 
 // The smoothstep argument of a lit pair at ISM texel (tx, ty), clamped to
@@ -273,7 +282,7 @@ __device__ __forceinline__ float shadow_arg(const LitConsts& lc, int ox, int oy,
 struct PairSetup {
   float g;         // clamped geometry term
   float sbase;     // 1 - dist / (bias zFar): the smoothstep argument without occ
-  uint32_t texel;  // ISM atlas texel (0 when shadowing is off)
+  uint32_t at;     // byte offset of the ISM atlas texel (0 when shadowing is off)
 };
 
 template <bool kMixed>
@@ -300,13 +309,14 @@ __device__ __forceinline__ PairSetup pair_setup(const GatherArgs& a, float px, f
     // back as GL_REPEAT does (final_gathering.comp:43-45, ism_utils.glsl:33-37)
     const int ism = vi - a.ism_offset;
     const int trow = (ism < 0 ? ism + a.n1d - 1 : ism) >> a.n1d_log2;
-    const int ox = (ism - trow * a.n1d) * a.ism_side;
+    const int tcol = ism - trow * a.n1d;
+    const int ox = tcol * a.ism_side;
     const int oy = trow * a.ism_side;
     r.sbase = __builtin_fmaf(-dist, lc.k1, 1.0f);
     int tx, ty;
     if (kMixed) {  // NEAREST decided in FP32 alone
-      tx = (int)floorf(cx);
-      ty = (int)floorf(cy);
+      tx = floor_int(cx);
+      ty = floor_int(cy);
     } else {
       const float fx = __builtin_amdgcn_fractf(cx), fy = __builtin_amdgcn_fractf(cy);
       tx = (int)(cx - fx);
@@ -329,7 +339,23 @@ __device__ __forceinline__ PairSetup pair_setup(const GatherArgs& a, float px, f
         }
       }
     }
-    r.texel = atlas_texel(lc, ox, oy, tx, ty);
+    if (kMixed) {
+      // A lit pair's texel lies in its VPL's tile or, on the horizon, one texel
+      // beside it, so only a tile on the atlas's border can wrap (a
+      // wave-uniform test): the others' texel is three instructions from
+      // (tx, ty) instead of six. This and floor_int take the lit path from 43
+      // to 38 of them (4K gather, bound by VALU issue: 500 -> 480 us with the
+      // square waves; 1080p 0.3 us). The FP32 form lost 1% with it. An index
+      // that is garbage (a non-finite position) reads 0 past the buffer's size.
+      const unsigned inner = (unsigned)(a.n1d - 2);
+      uint32_t origin = (uint32_t)((oy << lc.alog) + ox);
+      asm("" : "+s"(origin));  // one scalar sum: the compiler would add oy and ox per lane
+      r.at = (((uint32_t)ty << lc.alog) + (uint32_t)tx + origin) << 1;
+      if (__builtin_expect(!((unsigned)(tcol - 1) < inner && (unsigned)(trow - 1) < inner), 0))
+        r.at = atlas_texel(lc, ox, oy, tx, ty) << 1;
+    } else {
+      r.at = atlas_texel(lc, ox, oy, tx, ty) << 1;
+    }
   }
   return r;
 }
@@ -349,7 +375,7 @@ __device__ __forceinline__ float pair_weight(const GatherArgs& a, float px, floa
                                              float pdot, bool shadow, const LitConsts& lc) {
   const PairSetup s = pair_setup<kMixed>(a, px, py, pz, x, y, depth, vt, v, vi, ndot, pdot, shadow, lc);
   if (!shadow) return s.g;
-  return pair_finish(s, __builtin_amdgcn_raw_buffer_load_b16(lc.ism, s.texel << 1, 0, 0), lc);
+  return pair_finish(s, __builtin_amdgcn_raw_buffer_load_b16(lc.ism, s.at, 0, 0), lc);
 }
 
 // The flux half h of a record (binary16 bits) as a float: the conversion
@@ -481,7 +507,14 @@ __global__ __launch_bounds__(TW* TH) void final_gather_kernel(GatherArgs a, int 
   const int tile = w >> classes_log2;
   const int kx = k & (a.interleave - 1), ky = k >> a.interleave_log2;
   const int tile_x = tile % tiles_x, tile_y = tile / tiles_x;
-  const int lx = threadIdx.x % TW, ly = threadIdx.x / TW;
+  // A wave takes 8 x 8 of a tile whose sides allow it (16 x 16, 32 x 8: four
+  // such squares): its position box is the smallest there, so fewer VPLs
+  // survive the culling, and fewer light some lane of it (510 K wave-VPL pairs
+  // in rows of 16 x 4 at 1080p, 486 K in squares, counted on the CPU).
+  constexpr bool kSquares = TW % 8 == 0 && TH % 8 == 0;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int lx = kSquares ? (wave % (TW / 8)) * 8 + (lane & 7) : threadIdx.x % TW;
+  const int ly = kSquares ? (wave / (TW / 8)) * 8 + (lane >> 3) : threadIdx.x / TW;
   const Pixel p = load_pixel(a, tile_x * TW + lx, tile_y * TH + ly, kx, ky);
 
   // ---- wave bounds for culling
