@@ -7,8 +7,9 @@
 // in different slots run beside each other on the device. Each loop
 // iteration
 //   1. moves requests whose arrival time has passed into the FIFO queue,
-//   2. retires finished batches (event query), releasing their slots and
-//      arena ranges and recording completion times,
+//   2. retires finished batches (event query): moves their results from the
+//      slot's pinned staging buffer to the callers' memory, releases their
+//      slots and arena ranges and records completion times,
 //   3. if a queued-batch slot is free, admits queued requests in FIFO order
 //      while in-flight slots and arena space allow, renders each admitted
 //      request's RSM on the slot's stream and enqueues them there as one
@@ -24,10 +25,13 @@
 #include <algorithm>
 #include <chrono>
 #include <cmath>
+#include <condition_variable>
 #include <cstring>
 #include <deque>
 #include <iterator>
 #include <map>
+#include <memory>
+#include <mutex>
 #include <thread>
 #include <tuple>
 #include <utility>
@@ -93,6 +97,84 @@ class Arena {
   size_t size_ = 0, used_ = 0, peak_ = 0;
 };
 
+// Host copies from the pinned staging buffers to the callers' memory, in
+// pieces over a few threads: one thread's memcpy (~10 GB/s) took longer than
+// the device's work on a batch.
+class Copier {
+ public:
+  struct Job {
+    char* dst;
+    const char* src;
+    size_t bytes;
+  };
+  // As many helpers as can be started; with none, run() copies by itself.
+  explicit Copier(int helpers) {
+    try {
+      for (int i = 0; i < helpers; ++i) threads_.emplace_back([this] { help(); });
+    } catch (...) {
+    }
+  }
+  ~Copier() {
+    {
+      std::lock_guard<std::mutex> lock(mu_);
+      stop_ = true;
+    }
+    wake_.notify_all();
+    for (auto& t : threads_) t.join();
+  }
+  Copier(const Copier&) = delete;
+  Copier& operator=(const Copier&) = delete;
+  // Copies every job; the calling thread takes part and returns when all are done.
+  void run(const std::vector<Job>& jobs) {
+    std::unique_lock<std::mutex> lock(mu_);
+    for (const Job& j : jobs)
+      for (size_t o = 0; o < j.bytes; o += kPiece)
+        queue_.push_back({j.dst + o, j.src + o, std::min(kPiece, j.bytes - o)});
+    if (queue_.size() > 1) wake_.notify_all();
+    while (take(lock)) {
+    }
+    done_.wait(lock, [this] { return queue_.empty() && busy_ == 0; });
+  }
+
+ private:
+  static constexpr size_t kPiece = size_t(256) << 10;
+  // Copies one piece with the lock released; false when none is left.
+  bool take(std::unique_lock<std::mutex>& lock) {
+    if (queue_.empty()) return false;
+    const Job j = queue_.front();
+    queue_.pop_front();
+    ++busy_;
+    lock.unlock();
+    std::memcpy(j.dst, j.src, j.bytes);
+    lock.lock();
+    if (--busy_ == 0 && queue_.empty()) done_.notify_all();
+    return true;
+  }
+  void help() {
+    std::unique_lock<std::mutex> lock(mu_);
+    while (true) {
+      wake_.wait(lock, [this] { return stop_ || !queue_.empty(); });
+      if (stop_) return;
+      while (take(lock)) {
+      }
+    }
+  }
+  std::mutex mu_;
+  std::condition_variable wake_, done_;
+  std::deque<Job> queue_;
+  int busy_ = 0;
+  bool stop_ = false;
+  std::vector<std::thread> threads_;
+};
+
+// Pinned staging per batch slot for results on their way to the callers'
+// memory. A copy to pageable memory blocks the host until the batch's stream
+// has run dry, so no other batch is admitted or retired meanwhile; a copy to
+// pinned memory is queued. At most this much per slot and in all; results
+// that do not fit go directly, as all do where no memory can be pinned.
+constexpr size_t kStageSlotBytes = size_t(16) << 20, kStageBytes = size_t(96) << 20;
+constexpr int kCopyHelpers = 3;
+
 struct GBuf {
   float* depth = nullptr;
   float* normal = nullptr;
@@ -151,6 +233,7 @@ struct Inflight {
   hipEvent_t done;
   int ring;
   std::vector<Admitted> reqs;
+  std::vector<Copier::Job> staged;  // results that wait in the slot's staging buffer
 };
 
 }  // namespace
@@ -167,6 +250,9 @@ struct mlgi_server {
   // batch tables: ring of max_queued_batches slots of max_batch rows
   mlgi::BatchFrame* table_dev = nullptr;
   mlgi::BatchFrame* table_host = nullptr;  // pinned
+  char* stage = nullptr;                   // pinned, stage_bytes per slot
+  size_t stage_bytes = 0;
+  std::unique_ptr<Copier> copier;
   std::vector<hipEvent_t> events;
   std::vector<void*> owned;  // resident device allocations
   // one context (stream) per lane; lanes[0] is ctx, the others are owned
@@ -272,6 +358,7 @@ void mlgi_server_destroy(mlgi_server* s) {
   for (auto& sc : s->scenes) mlgi_scene_device_destroy(sc.dev);
   for (void* p : s->owned) (void)hipFree(p);
   if (s->table_host) (void)hipHostFree(s->table_host);
+  if (s->stage) (void)hipHostFree(s->stage);
   delete s;
 }
 
@@ -363,6 +450,19 @@ int mlgi_server_create(mlgi_context* c, const mlgi_server_config* cfg, const mlg
   if (!rc)
     rc = hip_check(c, hipHostMalloc((void**)&s->table_host, sizeof(mlgi::BatchFrame) * ring_rows, hipHostMallocDefault),
                    "hipHostMalloc");
+  if (!rc) {
+    size_t largest = 0;
+    for (auto& wh : s->resolutions) largest = std::max(largest, (size_t)wh.first * wh.second * 12);
+    s->stage_bytes = std::min(kStageSlotBytes, kStageBytes / (size_t)cfg->max_queued_batches);
+    s->stage_bytes = std::min(s->stage_bytes, largest * (size_t)cfg->max_batch);
+    if (hipHostMalloc((void**)&s->stage, s->stage_bytes * cfg->max_queued_batches, hipHostMallocDefault) !=
+        hipSuccess) {
+      (void)hipGetLastError();
+      s->stage = nullptr;
+      s->stage_bytes = 0;
+    }
+    s->copier.reset(new Copier(s->stage ? kCopyHelpers : 0));
+  }
   for (int i = 0; i < cfg->max_queued_batches && !rc; ++i) {
     hipEvent_t e = nullptr;
     rc = hip_check(c, hipEventCreateWithFlags(&e, hipEventDisableTiming), "hipEventCreate");
@@ -435,6 +535,7 @@ int mlgi_server_run(mlgi_server* s, const mlgi_request* reqs, int32_t n, mlgi_se
       const hipError_t q = hipEventQuery(inflight.front().done);
       if (q == hipErrorNotReady) break;
       if ((rc = hip_check(c, q, "hipEventQuery"))) break;
+      s->copier->run(inflight.front().staged);
       const double tc = now_s();
       for (const Admitted& a : inflight.front().reqs) {
         lat[a.req] = (tc - reqs[a.req].arrival_s) * 1e3;
@@ -455,6 +556,7 @@ int mlgi_server_run(mlgi_server* s, const mlgi_request* reqs, int32_t n, mlgi_se
       std::vector<Admitted> adm;
       std::vector<mlgi_frame_desc> descs;
       std::vector<mlgi_scene_impl::RsmJob> rsms;
+      std::vector<Copier::Job> staged;
       while (!queue.empty() && (int)adm.size() < s->cfg.max_batch && inflight_reqs < s->cfg.max_inflight) {
         const int i = queue.front();
         const mlgi_request& r = reqs[i];
@@ -499,17 +601,25 @@ int mlgi_server_run(mlgi_server* s, const mlgi_request* reqs, int32_t n, mlgi_se
                                            L->stream),
                          "hipMemcpyAsync(batch table)");
           if (!rc) rc = lane_fail(s, L, batch_enqueue(L, dev, plan));
+          char* stage = s->stage + (size_t)slot * s->stage_bytes;
+          size_t used = 0;
           for (const Admitted& a : adm) {
             if (rc || !reqs[a.req].host_out) continue;
             const size_t bytes = (size_t)reqs[a.req].width * reqs[a.req].height * 12;
-            rc = hip_check(c, hipMemcpyAsync(reqs[a.req].host_out, a.image, bytes, hipMemcpyDeviceToHost, L->stream),
+            char* dst = (char*)reqs[a.req].host_out;
+            if (used + bytes <= s->stage_bytes) {
+              staged.push_back({dst, stage + used, bytes});
+              dst = stage + used;
+              used += bytes;
+            }
+            rc = hip_check(c, hipMemcpyAsync(dst, a.image, bytes, hipMemcpyDeviceToHost, L->stream),
                            "hipMemcpyAsync(result)");
           }
           if (!rc) rc = hip_check(c, hipEventRecord(s->events[slot], L->stream), "hipEventRecord");
         }
         if (!rc) {
           if (!inflight.empty()) stats->overlapped_batches++;
-          inflight.push_back({s->events[slot], slot, std::move(adm)});
+          inflight.push_back({s->events[slot], slot, std::move(adm), std::move(staged)});
           stats->batches++;
           batched += (int64_t)inflight.back().reqs.size();
           stats->max_inflight_seen = std::max(stats->max_inflight_seen, inflight_reqs);
