@@ -170,8 +170,9 @@ class Copier {
 // Pinned staging per batch slot for results on their way to the callers'
 // memory. A copy to pageable memory blocks the host until the batch's stream
 // has run dry, so no other batch is admitted or retired meanwhile; a copy to
-// pinned memory is queued. At most this much per slot and in all; results
-// that do not fit go directly, as all do where no memory can be pinned.
+// pinned memory is queued (a burst of 24 requests: 4.25 ms direct, 2.36 ms
+// staged). At most this much per slot and in all; results that do not fit go
+// directly, as all do where no memory can be pinned.
 constexpr size_t kStageSlotBytes = size_t(16) << 20, kStageBytes = size_t(96) << 20;
 constexpr int kCopyHelpers = 3;
 
@@ -235,6 +236,32 @@ struct Inflight {
   std::vector<Admitted> reqs;
   std::vector<Copier::Job> staged;  // results that wait in the slot's staging buffer
 };
+
+// Which results may wait in staging: those bound for ordinary memory that no
+// other request of the run writes. Memory that HIP knows (pinned, managed, on
+// a device) takes a queued copy as it is and need not be reachable by the
+// host; results that share memory keep the order of their streams' copies.
+std::vector<char> stageable(const mlgi_request* reqs, int n) {
+  std::vector<char> yes((size_t)n, 0);
+  std::vector<std::tuple<uintptr_t, uintptr_t, int>> range;  // begin, end, request
+  for (int i = 0; i < n; ++i) {
+    if (!reqs[i].host_out) continue;
+    hipPointerAttribute_t at{};
+    const hipError_t e = hipPointerGetAttributes(&at, reqs[i].host_out);
+    if (e != hipSuccess) (void)hipGetLastError();
+    yes[i] = e == hipErrorInvalidValue || (e == hipSuccess && at.type == hipMemoryTypeUnregistered);
+    const uintptr_t b = (uintptr_t)reqs[i].host_out;
+    range.emplace_back(b, b + (uintptr_t)reqs[i].width * reqs[i].height * 12, i);
+  }
+  std::sort(range.begin(), range.end());
+  size_t last = 0;  // the range that ends furthest so far
+  for (size_t k = 1; k < range.size(); ++k) {
+    if (std::get<0>(range[k]) < std::get<1>(range[last]))
+      yes[std::get<2>(range[k])] = yes[std::get<2>(range[last])] = 0;
+    if (std::get<1>(range[k]) > std::get<1>(range[last])) last = k;
+  }
+  return yes;
+}
 
 }  // namespace
 
@@ -514,6 +541,8 @@ int mlgi_server_run(mlgi_server* s, const mlgi_request* reqs, int32_t n, mlgi_se
       return fail(c, MLGI_ERR_INVALID_ARGUMENT, "requests must be sorted by arrival");
   }
   std::memset(stats, 0, sizeof *stats);
+  std::vector<char> may_stage(n, 0);
+  if (s->stage) may_stage = stageable(reqs, n);
   std::vector<double> lat(n, -1.0);
   std::deque<int> queue;
   std::deque<Inflight> inflight;
@@ -607,7 +636,7 @@ int mlgi_server_run(mlgi_server* s, const mlgi_request* reqs, int32_t n, mlgi_se
             if (rc || !reqs[a.req].host_out) continue;
             const size_t bytes = (size_t)reqs[a.req].width * reqs[a.req].height * 12;
             char* dst = (char*)reqs[a.req].host_out;
-            if (used + bytes <= s->stage_bytes) {
+            if (may_stage[a.req] && used + bytes <= s->stage_bytes) {
               staged.push_back({dst, stage + used, bytes});
               dst = stage + used;
               used += bytes;
@@ -629,7 +658,10 @@ int mlgi_server_run(mlgi_server* s, const mlgi_request* reqs, int32_t n, mlgi_se
     }
     if (!progress) std::this_thread::yield();
   }
-  for (mlgi_context* L : s->lanes) (void)hipStreamSynchronize(L->stream);
+  bool drained = true;
+  for (mlgi_context* L : s->lanes) drained &= hipStreamSynchronize(L->stream) == hipSuccess;
+  for (Inflight& b : inflight)  // left only by an error: what did finish is delivered
+    if (drained) s->copier->run(b.staged);
   if (rc) return rc;
   std::vector<double> ok;
   for (int i = 0; i < n; ++i)
