@@ -1382,16 +1382,27 @@ int mlgi_scene_device_sample_points(mlgi_context* c, const mlgi_scene_device* d,
                 n_bins, ism_count);
   const int n = (int)n_points;
   const float r_packed = mlgi_scene_point_radius(d->total_area, n_points, ism_count);
-  // one work area: records, places, counts
+  // one work area: records, places, counts, and a row of counts per workgroup
+  // where there is room for it
   const size_t rec_bytes = sizeof(float) * 4 * (size_t)n, place_bytes = sizeof(uint2) * (size_t)n;
+  const size_t count_bytes = sizeof(uint32_t) * (size_t)n_bins;
+  const size_t hist_bytes = count_bytes * (size_t)mlgi::points_hist_rows(n, n_bins);
   char* work = nullptr;
-  int rc = hip_check(c, hipMalloc(&work, rec_bytes + place_bytes + sizeof(uint32_t) * (size_t)n_bins),
-                     "hipMalloc(points work)");
+  uint32_t* hist = nullptr;
+  int rc = MLGI_OK;
+  if (hist_bytes && hipMalloc(&work, rec_bytes + place_bytes + count_bytes + hist_bytes) == hipSuccess) {
+    hist = (uint32_t*)(work + rec_bytes + place_bytes + count_bytes);
+  } else {
+    if (hist_bytes) (void)hipGetLastError();
+    work = nullptr;
+    rc = hip_check(c, hipMalloc(&work, rec_bytes + place_bytes + count_bytes), "hipMalloc(points work)");
+  }
   if (!rc)
     rc = hip_check(c,
                    mlgi::launch_sample_points(c->stream, d->tris, d->cdf, d->n_tris, d->total_area, seed, r_packed,
                                               n_bins, n, (float*)work, (uint2*)(work + rec_bytes),
-                                              (uint32_t*)(work + rec_bytes + place_bytes), records, bin_offsets),
+                                              (uint32_t*)(work + rec_bytes + place_bytes), hist, records,
+                                              bin_offsets),
                    "sample_points");
   if (!rc) rc = hip_check(c, hipStreamSynchronize(c->stream), "hipStreamSynchronize");
   if (work) (void)hipFree(work);

@@ -138,10 +138,12 @@ struct Tri;
 }  // namespace mlgi_scene_impl
 namespace mlgi {
 // points.hip: device point set of a scene (records grouped by bin). Work
-// buffers: tmp (4n floats), place (n: bin, place in the bin), count (n_bins).
+// buffers: tmp (4n floats), place (n: bin, place in the bin), count (n_bins),
+// hist (points_hist_rows() x n_bins; NULL: places from atomics in memory).
+int points_hist_rows(int n, int n_bins);
 hipError_t launch_sample_points(hipStream_t s, const mlgi_scene_impl::Tri* tris, const double* cdf, int nt,
                                 double total, uint64_t seed, float r_packed, int n_bins, int n, float* tmp,
-                                uint2* place, uint32_t* count, float* records, uint32_t* offsets);
+                                uint2* place, uint32_t* count, uint32_t* hist, float* records, uint32_t* offsets);
 // n RSMs of w x h texels, up to kRsmJobs of them in one launch: one 128^2 RSM
 // is a wave per SIMD bound by its longest packet, and others fit beside it.
 hipError_t launch_rsms(hipStream_t st, const mlgi_scene_impl::RsmJob* jobs, int n, int w, int h);

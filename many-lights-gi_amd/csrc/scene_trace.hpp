@@ -395,10 +395,12 @@ MLGI_HD inline int upper_bound_d(const double* cdf, int n, double u) {
 // Point i: a triangle drawn by area, a uniform point on it, its record
 // (pos, packUnorm4x8(n * 0.5 + 0.5, r / 25)) and its bin
 // int(random(pos) * n_bins), clamped to [0, n_bins).
-MLGI_HD inline void sample_point(const Tri* tris, const double* cdf, int nt, double total, uint64_t seed,
-                                 uint64_t i, float r_packed, int n_bins, float rec[4], int* bin) {
-  const double u0 = counter_uniform(seed, i, 0) * total;
-  int ti = upper_bound_d(cdf, nt, u0);
+// ti: the first triangle whose running area exceeds point_area(), or nt.
+MLGI_HD inline double point_area(double total, uint64_t seed, uint64_t i) {
+  return counter_uniform(seed, i, 0) * total;
+}
+MLGI_HD inline void sample_on(const Tri* tris, int ti, int nt, uint64_t seed, uint64_t i, float r_packed, int n_bins,
+                              float rec[4], int* bin) {
   if (ti >= nt) ti = nt - 1;
   const Tri& tr = tris[ti];
   const double r1 = sqrt(counter_uniform(seed, i, 1));
@@ -413,6 +415,10 @@ MLGI_HD inline void sample_point(const Tri* tris, const double* cdf, int nt, dou
   rec[3] = __builtin_bit_cast(float, bits);
   const int bi = (int)(glsl_random3(px, py, pz) * (float)n_bins);
   *bin = bi < 0 ? 0 : (bi > n_bins - 1 ? n_bins - 1 : bi);
+}
+MLGI_HD inline void sample_point(const Tri* tris, const double* cdf, int nt, double total, uint64_t seed,
+                                 uint64_t i, float r_packed, int n_bins, float rec[4], int* bin) {
+  sample_on(tris, upper_bound_d(cdf, nt, point_area(total, seed, i)), nt, seed, i, r_packed, n_bins, rec, bin);
 }
 
 }  // namespace mlgi_scene_impl
