@@ -84,9 +84,8 @@ constexpr int kBatchXcds = 8;
 // 108 with 4. One frame: 1080p tiles 30.0 (eighths), 29.4 (32), 30.2 (4); 4K
 // 99.8, 97.7, 103.0.
 __host__ __device__ inline uint32_t xcd_chunk_log2(uint32_t items) {
-  uint32_t l = 0;
-  while (l < 5 && (items >> (l + 6)) != 0) ++l;
-  return l;
+  const uint32_t l = 31u - (uint32_t)__builtin_clz(items | 32u);  // floor(log2), at least 5
+  return l > 10u ? 5u : l - 5u;
 }
 __device__ __forceinline__ uint32_t xcd_item(uint32_t items) {
   const uint32_t l = xcd_chunk_log2(items);

@@ -1015,8 +1015,9 @@ int batch_frame(mlgi_context* c, const mlgi_frame_desc& d, mlgi::BatchFrame* f) 
   a.out = d.image.rgb;
   a.ism = d.ism.texels;  // the pull-push writes it even when the gather does not shadow
   f->g = a;
-  // a 16 x 16 tile is four 8 x 8 waves, as in the single-frame kernel
-  const int wave_w = tw == 16 && p->tile_h == 16 ? 8 : tw;
+  // a 16 x 16 tile is four 8 x 8 waves where it shadows, as in the
+  // single-frame kernel
+  const int wave_w = tw == 16 && p->tile_h == 16 && a.shadowing ? 8 : tw;
   f->wave_w_log2 = log2i(wave_w);
   const int cw = (a.width + a.interleave - 1) / a.interleave;
   f->strips_x = (cw + wave_w - 1) / wave_w;
