@@ -434,7 +434,22 @@ __device__ __forceinline__ void kahan_add(float& total, float& comp, float x) {
 //   kFetchWhole     the full record at the top of each iteration
 //   kFetchTestFirst the hemisphere-test fields per iteration, the rest only
 //                   when a lane is lit
-enum FetchVariant { kFetchWhole = 0, kFetchTestFirst = 1 };
+// and, in place of kFetchWhole where few waves hide its latency (ahead_pays),
+//   kFetchAhead     the full record of the next survivor, requested before the
+//                   current pair is evaluated
+enum FetchVariant { kFetchWhole = 0, kFetchTestFirst = 1, kFetchAhead = 2 };
+
+// FP32 launches of few waves wait for each record in turn. With many, others
+// run meanwhile, and the second record's scalar registers and moves cost more.
+// Whole / ahead over interleaves of 2 to 8 and tiles of 8 x 8 and 16 x 16:
+// shadowed, 96 to 1,024 waves 1.01 to 1.22, 1,300 0.96 to 1.06, 1,600 0.94 to
+// 1.03, 4,000 0.85 to 0.93 (96 x 64 in classes of 4 x 4, 64 VPLs each: 29.3 ->
+// 24.4 us); unshadowed, 96 to 1,600 1.10 to 1.38, 4,000 0.98 to 1.09. The mixed
+// form is 2% slower with it, shadowed, at any size.
+constexpr uint32_t kAheadWaves = 2048, kAheadWavesShadow = 1024;
+inline bool ahead_pays(bool mixed, bool shadow, uint32_t waves) {
+  return !mixed && waves <= (shadow ? kAheadWavesShadow : kAheadWaves);
+}
 
 // Precision forms.
 //   FP32  the reference's arithmetic in FP32, NEAREST texel decisions that
@@ -464,13 +479,19 @@ __device__ __forceinline__ void class_sums(const GatherArgs& a, const Pixel& p, 
     const int count = min(64, a.per_class - chunk);
     const float* crec = a.vpl + (size_t)(first + chunk) * kVplFloats;
     unsigned long long mask = cull_chunk<kMixed>(crec, count, wb, a.cull);
+    VplLds ahead;
+    if (kFetch == kFetchAhead && mask) ahead = uniform_vpl(a.vpl, first + chunk + __builtin_ctzll(mask));
     while (mask) {
       const int j = __builtin_ctzll(mask);
       mask &= mask - 1ull;
       const int vi = first + chunk + j;
       VplTest vt;
       VplLds vf;
-      if (kFetch == kFetchWhole) {
+      if (kFetch == kFetchAhead) {
+        vf = ahead;
+        vt = VplTest{vf.px, vf.py, vf.pz, vf.plane, vf.nx, vf.ny, vf.nz};
+        ahead = uniform_vpl(a.vpl, mask ? first + chunk + __builtin_ctzll(mask) : vi);
+      } else if (kFetch == kFetchWhole) {
         vf = uniform_vpl(a.vpl, vi);
         vt = VplTest{vf.px, vf.py, vf.pz, vf.plane, vf.nx, vf.ny, vf.nz};
       } else {
@@ -562,11 +583,9 @@ __global__ __launch_bounds__(TW* TH) void final_gather_kernel(GatherArgs a, int 
 // chunk's culling records before the pixel loads, to overlap the two
 // latencies, measured 9% slower at 4K and 15% slower for FP32: the records
 // stay live across the pixel reconstruction and the bound reductions.)
-// Occupancy: eight waves per SIMD (64 VGPRs) for MIXED; the FP32 form's
-// exact-texel path needs 67, which spill at eight.
-template <bool kMixed>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kMixed ? 8 : 7))) void batch_gather_kernel(const BatchFrame* __restrict__ frames, int n,
-                                                           uint32_t total, int chunk_log2) {
+template <bool kMixed, int kFetch>
+__device__ __forceinline__ void batch_gather(const BatchFrame* __restrict__ frames, int n, uint32_t total,
+                                             int chunk_log2) {
   const int lane = threadIdx.x;
   // One single-wave workgroup per item, dispatched by the hardware as waves
   // retire (a persistent grid walking the items ran the same instructions
@@ -600,11 +619,11 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kMixed ? 8 :
     float ar = 0.0f, ag = 0.0f, ab = 0.0f;
     // the frame's shadowing flag picks one of two instances of the VPL loop
     // (a scalar branch), so that the lit path holds no per-lane copy of it;
-    // the loop is the single-frame kernel's with the whole-record fetch
+    // the loop is the single-frame kernel's
     if (__builtin_amdgcn_readfirstlane(a.shadowing))
-      class_sums<kMixed, true, kFetchWhole>(a, p, wb, first, lc, ar, ag, ab);
+      class_sums<kMixed, true, kFetch>(a, p, wb, first, lc, ar, ag, ab);
     else
-      class_sums<kMixed, false, kFetchWhole>(a, p, wb, first, lc, ar, ag, ab);
+      class_sums<kMixed, false, kFetch>(a, p, wb, first, lc, ar, ag, ab);
     if (p.valid) {
       float* o = a.out + ((size_t)p.y * a.width + p.x) * 3;
       gstore(o, ar * a.out_scale);
@@ -612,6 +631,20 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kMixed ? 8 :
       gstore(o + 2, ab * a.out_scale);
     }
   }
+}
+
+// Occupancy: eight waves per SIMD (64 VGPRs) for MIXED; the FP32 form's
+// exact-texel path needs 67, which spill at eight.
+template <bool kMixed>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(kMixed ? 8 : 7))) void batch_gather_kernel(
+    const BatchFrame* __restrict__ frames, int n, uint32_t total, int chunk_log2) {
+  batch_gather<kMixed, kFetchWhole>(frames, n, total, chunk_log2);
+}
+// FP32 launches of few waves (ahead_pays): a 96 x 64 frame 37.4 -> 36.5 us, a
+// 256 x 200 one 62.5 -> 61.8.
+__global__ __launch_bounds__(64) void batch_gather_ahead_kernel(const BatchFrame* __restrict__ frames, int n,
+                                                                uint32_t total, int chunk_log2) {
+  batch_gather<false, kFetchAhead>(frames, n, total, chunk_log2);
 }
 
 // Lit-pair counter: pairs (pixel, VPL of its class) with angleFactor > 0,
@@ -650,6 +683,10 @@ hipError_t launch_tiled(hipStream_t s, const GatherArgs& a) {
   const int num_work = tiles_x * tiles_y * a.interleave * a.interleave;
   const int per_xcd = (num_work + kXcds - 1) / kXcds;
   const dim3 grid(per_xcd * kXcds), block(TW * TH);
+  if constexpr (kFetch == kFetchWhole && !kMixed) {
+    if (ahead_pays(kMixed, a.shadowing, (uint32_t)num_work * (TW * TH / 64)))
+      return launch_tiled<TW, TH, kFetchAhead, kMixed>(s, a);
+  }
   if (a.shadowing)
     hipLaunchKernelGGL((final_gather_kernel<TW, TH, true, kFetch, kMixed>), grid, block, 0, s, a,
                        tiles_x, num_work, per_xcd);
@@ -697,6 +734,8 @@ hipError_t launch_batch_gather(hipStream_t s, const BatchFrame* frames, int n, u
   const unsigned grid = (unsigned)((total + per_round - 1) / per_round * per_round);
   if (precision == 1)
     hipLaunchKernelGGL(batch_gather_kernel<true>, dim3(grid), dim3(64), 0, s, frames, n, total, chunk_log2);
+  else if (ahead_pays(false, true, total))
+    hipLaunchKernelGGL(batch_gather_ahead_kernel, dim3(grid), dim3(64), 0, s, frames, n, total, chunk_log2);
   else
     hipLaunchKernelGGL(batch_gather_kernel<false>, dim3(grid), dim3(64), 0, s, frames, n, total, chunk_log2);
   return hipGetLastError();

@@ -48,3 +48,33 @@ def test_tile_shapes_and_wraps(ctx, n_vpl, interleave, atlas, size, precision, b
     norm = np.linalg.norm(ref)
     for im in images[:2]:
         assert np.linalg.norm(im - ref) <= bar * norm
+
+
+@pytest.mark.parametrize("shadowing", [True, False])
+@pytest.mark.parametrize("size", [(33, 17), (256, 256), (260, 256), (352, 362), (362, 362)])
+def test_record_fetch_forms(ctx, size, shadowing):
+    """FP32: the next record requested ahead (launches of few waves; the sizes
+    lie around 1,024 and 2,048 waves), each record requested in turn, and the
+    batched kernel give the same bits."""
+    print(f"[gather] fetch forms {size} shadowing={shadowing}", flush=True)
+    wl = W.WORKLOADS["tiny"].with_(n_vpl=1024, interleave=2, atlas_side=512, width=size[0], height=size[1],
+                                   n_points=6_000, levels=2)
+    inp = W.build_inputs(wl)
+    rsm = mlgi.rsm_desc(ctx.upload(inp.rsm_diffuse), ctx.upload(inp.rsm_normal), ctx.upload(inp.rsm_depth), inp.inv_bvp)
+    pts = mlgi.points_desc(ctx.upload(inp.points), ctx.upload(inp.bin_offsets))
+    gb = mlgi.gbuffer_desc(ctx.upload(inp.gb_depth), ctx.upload(inp.gb_normal), inp.vp_inv)
+    images = []
+    for fetch in (0, 1):
+        p = wl.params(precision=mlgi.PRECISION_FP32)
+        p.tile_w, p.tile_h, p.gather_fetch, p.enable_shadowing = 8, 8, fetch, int(shadowing)
+        st = mlgi.GIStage(ctx, p, wl.n_vpl, *size)
+        st.process(rsm, pts, gb)
+        ctx.sync()
+        images.append(st.gi_buffer.numpy())
+    b = mlgi.Batch(ctx, [(st, rsm, pts, gb)])
+    b.run()
+    ctx.sync()
+    images.append(st.gi_buffer.numpy())
+    b.close()
+    assert images[0].max() > 0
+    assert np.array_equal(images[0], images[1]) and np.array_equal(images[0], images[2])
