@@ -22,7 +22,7 @@
 // places), and is formed once for the pairs within a run, the three channels'
 // quotients share one reciprocal, a taller tile's apron costs fewer extra rows
 // (1.375 per row at 16, 1.75 at 8), and all loads of a tile are in flight at
-// once: 25.6 us at 1080p, and down to 130 x 109 no slower than the smaller
+// once: 25.1 us at 1080p, and down to 130 x 109 no slower than the smaller
 // forms. Other forms at 1080p: 32 x 16 tiles with one pixel per lane 27.9,
 // with two 28.1, with four 38.5 (a third of the waves); 32 x 8 with one 32.9.
 #include "kernels.hpp"
@@ -186,9 +186,9 @@ __global__ __launch_bounds__(kThreads) void gi_blur_kernel(const float* __restri
       const int y = y0 + ty + o;
       if (x < w && y < h) {
         float* p = out + ((size_t)y * w + x) * 3;
-        p[0] = r[o][0];
-        p[1] = r[o][1];
-        p[2] = r[o][2];
+        __builtin_nontemporal_store(r[o][0], p);  // 25.6 -> 25.1 us at 1080p: a stream past the L2s
+        __builtin_nontemporal_store(r[o][1], p + 1);
+        __builtin_nontemporal_store(r[o][2], p + 2);
       }
     }
   }
