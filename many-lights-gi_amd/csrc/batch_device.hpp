@@ -42,11 +42,6 @@ __device__ __forceinline__ uint4 gload4(const uint4* p) {
   const v4u v = *(const __attribute__((address_space(1))) v4u*)p;
   return make_uint4(v.x, v.y, v.z, v.w);
 }
-__device__ __forceinline__ void gstore4(uint4* p, uint4 v) {
-  typedef unsigned int v4u __attribute__((ext_vector_type(4)));
-  v4u w = {v.x, v.y, v.z, v.w};
-  *(__attribute__((address_space(1))) v4u*)p = w;
-}
 // Relaxed, agent-scope atomics on global memory (no return value needed
 // except for the add).
 __device__ __forceinline__ uint32_t gatomic_add(uint32_t* p, uint32_t v) {

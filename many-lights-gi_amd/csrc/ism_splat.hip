@@ -321,6 +321,32 @@ struct TileJob {
   uint2* spill;
 };
 
+// How a finished tile is stored. Plain stores leave up to 32 MB of it dirty in
+// the eight L2s, which the end of the kernel waits for. Write-through stores
+// (agent scope, sc1) go to memory as they are issued and leave the atlas in the
+// last-level cache for the pull-push: 1080p frame 187.0 -> 185.7 us, splat and
+// pull-push of a 2,048^2 atlas 45.4 -> 43.5. From kStreamBytes of atlas in a
+// launch on it would have left that cache (256 MB) before the pull-push comes;
+// stored as a stream (nt) it does not push the points and masks out either.
+// Write-through / stream, us: batches with 68 MB of tiles 201/203, 132 MB
+// 262/270, 196 MB 381/370, 329 MB 582/557, 403 MB 814/776.
+constexpr uint64_t kStreamBytes = uint64_t(176) << 20;
+constexpr int kAuxStream = 2, kAuxWriteThrough = 16;  // nt, sc1
+
+template <int kAux>
+__device__ __forceinline__ void store_tile(const TileJob& j, const uint4* t4, size_t origin) {
+  typedef unsigned int v4u __attribute__((ext_vector_type(4)));
+  const int S = j.ism_side;
+  const __amdgpu_buffer_rsrc_t to =
+      __builtin_amdgcn_make_buffer_rsrc(j.atlas, 0, (int)((uint32_t)j.atlas_side * (uint32_t)j.atlas_side * 4u), 0x00020000);
+  for (int i = threadIdx.x; i < S * S / 4; i += 256) {
+    const uint32_t row = (uint32_t)(i * 4) / (uint32_t)S, col = (uint32_t)(i * 4) % (uint32_t)S;
+    const uint4 t = t4[i];
+    __builtin_amdgcn_raw_buffer_store_b128(v4u{t.x, t.y, t.z, t.w}, to,
+                                           (int)(((uint32_t)origin + row * (uint32_t)j.atlas_side + col) * 4u), 0, kAux);
+  }
+}
+
 // One queued point splatted into ISM c (tile origin ox, oy).
 __device__ __forceinline__ void splat_queued(const TileJob& j, uint32_t* tile, const Candidate& c, float4 rec,
                                              uint32_t ox, uint32_t oy, float inv_n1d, float side) {
@@ -342,7 +368,7 @@ __device__ __forceinline__ void splat_queued(const TileJob& j, uint32_t* tile, c
 // Tile pass of ISM v (all 256 lanes; ends after the tile is written). `tile`
 // holds at least S * S words, `queues` 4 * kQueue<QueueT> entries.
 template <class QueueT>
-__device__ __forceinline__ void splat_tile(const TileJob& j, uint32_t* tile, QueueT* queues, int v) {
+__device__ __forceinline__ void splat_tile(const TileJob& j, uint32_t* tile, QueueT* queues, int v, bool stream) {
   constexpr bool kCoded = sizeof(QueueT) == 2;
   constexpr int kSt = kStep<QueueT>, kLoads = kSt / 64;
   const int tid = threadIdx.x, lane = tid & 63;
@@ -443,10 +469,10 @@ __device__ __forceinline__ void splat_tile(const TileJob& j, uint32_t* tile, Que
   }
   __syncthreads();
   const size_t origin = (size_t)tile_y * S * j.atlas_side + (size_t)tile_x * S;
-  for (int i = tid; i < n4; i += 256) {
-    const int row = (i * 4) / S, col = (i * 4) % S;
-    gstore4(reinterpret_cast<uint4*>(j.atlas + origin + (size_t)row * j.atlas_side + col), t4[i]);
-  }
+  if (stream)
+    store_tile<kAuxStream>(j, t4, origin);
+  else
+    store_tile<kAuxWriteThrough>(j, t4, origin);
 }
 
 // Workgroups of the spill pass.
@@ -497,11 +523,11 @@ __global__ __launch_bounds__(256) void ism_mask_kernel(TileJob j, int n_bins) {
 }
 
 template <class QueueT>
-__global__ __launch_bounds__(256) void ism_tiles_kernel(TileJob j, int n_tiles) {
+__global__ __launch_bounds__(256) void ism_tiles_kernel(TileJob j, int n_tiles, bool stream) {
   QueueT* queues = reinterpret_cast<QueueT*>(tile_lds + j.ism_side * j.ism_side);
   const uint32_t v = xcd_item((uint32_t)n_tiles);
   if (v >= (uint32_t)n_tiles) return;
-  splat_tile(j, tile_lds, queues, (int)v);
+  splat_tile(j, tile_lds, queues, (int)v, stream);
 }
 
 __global__ __launch_bounds__(256) void ism_spill_kernel(TileJob j, int n_bins) {
@@ -524,12 +550,12 @@ __global__ __launch_bounds__(256) void batch_mask_kernel(const BatchFrame* __res
 
 template <class QueueT>
 __global__ __launch_bounds__(256) void batch_tiles_kernel(const BatchFrame* __restrict__ frames, int n,
-                                                          uint32_t total, int max_side) {
+                                                          uint32_t total, int max_side, bool stream) {
   QueueT* queues = reinterpret_cast<QueueT*>(tile_lds + max_side * max_side);
   const uint32_t item = xcd_item(total);
   if (item >= total) return;
   const BatchFrame& f = frames[batch_find<&BatchFrame::first_tile>(frames, n, item)];
-  splat_tile(tile_job(f), tile_lds, queues, (int)(item - f.first_tile));
+  splat_tile(tile_job(f), tile_lds, queues, (int)(item - f.first_tile), stream);
 }
 
 // Batched spill: the frames one after the other, each by the whole grid.
@@ -633,11 +659,14 @@ hipError_t launch_ism_splat_tiled(hipStream_t s, const float* points, const uint
     if (e != hipSuccess) return e;
   }
   const int n_tiles = n1d * n1d;
+  const bool stream = (uint64_t)n_tiles * ism_side * ism_side * 4 >= kStreamBytes;
   const dim3 grid(xcd_items_grid((uint32_t)n_tiles));
   if (ism_side > 32)
-    hipLaunchKernelGGL(ism_tiles_kernel<uint16_t>, grid, dim3(256), tile_lds_bytes<uint16_t>(ism_side), s, j, n_tiles);
+    hipLaunchKernelGGL(ism_tiles_kernel<uint16_t>, grid, dim3(256), tile_lds_bytes<uint16_t>(ism_side), s, j, n_tiles,
+                       stream);
   else
-    hipLaunchKernelGGL(ism_tiles_kernel<uint32_t>, grid, dim3(256), tile_lds_bytes<uint32_t>(ism_side), s, j, n_tiles);
+    hipLaunchKernelGGL(ism_tiles_kernel<uint32_t>, grid, dim3(256), tile_lds_bytes<uint32_t>(ism_side), s, j, n_tiles,
+                       stream);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || !any) return e;
   // a few entries in the normal case: one workgroup per CU at most (the
@@ -679,12 +708,13 @@ hipError_t launch_batch_tiles(hipStream_t s, const BatchFrame* frames, int n, ui
   if (total == 0) return hipSuccess;
   if (max_side < 4 || max_side > kTileMax) return hipErrorInvalidValue;
   const dim3 grid(xcd_items_grid(total));
+  const bool stream = (uint64_t)total * max_side * max_side * 4 >= kStreamBytes;
   if (max_side > 32)
     hipLaunchKernelGGL(batch_tiles_kernel<uint16_t>, grid, dim3(256), tile_lds_bytes<uint16_t>(max_side), s, frames, n,
-                       total, max_side);
+                       total, max_side, stream);
   else
     hipLaunchKernelGGL(batch_tiles_kernel<uint32_t>, grid, dim3(256), tile_lds_bytes<uint32_t>(max_side), s, frames, n,
-                       total, max_side);
+                       total, max_side, stream);
   return hipGetLastError();
 }
 
