@@ -142,6 +142,7 @@ __global__ __launch_bounds__(256) void composite_kernel(CompositeArgs a) {
   const float occ = a.occlusion ? a.occlusion[c] : 1.0f;
   const float h1 = fmaxf(0.0f, ndoth), h2 = h1 * h1, h4 = h2 * h2, h5 = h4 * h1, h10 = h5 * h5;
   const float spec_f = h10 * h10;  // (n . h)^20
+  float res[3];
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
     const float dif = pow_pos(a.diffuse[c * 3 + k], 2.2f);
@@ -153,8 +154,14 @@ __global__ __launch_bounds__(256) void composite_kernel(CompositeArgs a) {
     // from 2^30 on 1 + col is col; an infinite or NaN col divides to NaN, which
     // the power makes 0
     const float cap = fminf(col, 0x1p30f);
-    a.out[c * 3 + k] = col < __builtin_inff() ? pow_pos(quotient(cap, 1.0f + cap), 1.0f / 2.2f) : 0.0f;
+    res[k] = col < __builtin_inff() ? pow_pos(quotient(cap, 1.0f + cap), 1.0f / 2.2f) : 0.0f;
   }
+  // together, so that no channel's loads wait behind another's store (41.3 ->
+  // 37.0 us at 1080p), and as a stream past the L2s (35.6)
+  float* o = a.out + c * 3;
+  __builtin_nontemporal_store(res[0], o);
+  __builtin_nontemporal_store(res[1], o + 1);
+  __builtin_nontemporal_store(res[2], o + 2);
 }
 
 }  // namespace
