@@ -10,7 +10,7 @@
 // Bound: with the library's powf (ten per pixel) and IEEE division sequences
 // (17) it was VALU issue, 82 us for 1080p. The quotients are formed from the
 // correctly rounded reciprocals of their divisors (dev::div_rn: the same bits;
-// divisors outside its range take the division), the three divisions by one
+// operands outside its range take the division), the three divisions by one
 // length or w share one reciprocal, and the powers of the gamma are formed
 // from the hardware's base-2 logarithm and exponential (pow_pos).
 //
@@ -40,14 +40,17 @@ __device__ __forceinline__ void divide(float& a, float& b, float& c, float d) {
     a = a / d, b = b / d, c = c / d;
   }
 }
-// a / b where b is known to be a plain number, or a NaN does as well as the
-// quotient.
+// a / b for plain numbers.
 __device__ __forceinline__ float quotient(float a, float b) { return dev::div_rn(a, b, dev::recip_rn(b)); }
+// a / b for any: an infinite moment or colour, a window or sum that is 0 or
+// huge take the division, whose infinities the clamps turn into 0 or 1.
+__device__ __forceinline__ float quotient_any(float a, float b) {
+  const float m = fabsf(b);
+  return m >= 0x1p-40f && m <= 0x1p40f && fabsf(a) <= 0x1p60f ? quotient(a, b) : a / b;
+}
 
 __device__ __forceinline__ float smoothstep_f(float e0, float e1, float x) {
-  // far from the light e1 - e0 rounds to 0: the division gives +-inf or NaN
-  const float w = e1 - e0;
-  const float t = w == 0.0f ? (x > e0 ? 1.0f : 0.0f) : clamp01(quotient(x - e0, w));
+  const float t = clamp01(quotient_any(x - e0, e1 - e0));
   return t * t * (3.0f - 2.0f * t);
 }
 
@@ -75,8 +78,7 @@ __device__ __forceinline__ float vsm_factor(float mx, float my, float compare) {
   // E[d^2] - E[d]^2 cancels: one rounding (fused) instead of two
   const float variance = fmaxf(__builtin_fmaf(-mx, mx, my), 0.001f);
   const float d = compare - mx;
-  // a NaN quotient (an infinite d * d) clamps to 0, as the 0 it stands for
-  const float p_max = clamp01(quotient(quotient(variance, variance + d * d) - 0.1f, 1.0f - 0.1f));
+  const float p_max = clamp01(quotient(quotient_any(variance, variance + d * d) - 0.1f, 1.0f - 0.1f));
   return clamp01(fmaxf(p, p_max));
 }
 
@@ -150,11 +152,8 @@ __global__ __launch_bounds__(256) void composite_kernel(CompositeArgs a) {
     const float ambient = a.gi[c * 3 + k] * dif * occ;
     const float dterm = dif * (fmaxf(0.0f, ndotl) * shadow) * a.light_intensity;
     const float sterm = 0.75f * spc * spec_f * shadow;
-    float col = (ambient + dterm + sterm) * a.exposure;
-    // from 2^30 on 1 + col is col; an infinite or NaN col divides to NaN, which
-    // the power makes 0
-    const float cap = fminf(col, 0x1p30f);
-    res[k] = col < __builtin_inff() ? pow_pos(quotient(cap, 1.0f + cap), 1.0f / 2.2f) : 0.0f;
+    const float col = (ambient + dterm + sterm) * a.exposure;
+    res[k] = pow_pos(quotient_any(col, 1.0f + col), 1.0f / 2.2f);
   }
   // together, so that no channel's loads wait behind another's store (41.3 ->
   // 37.0 us at 1080p), and as a stream past the L2s (35.6)
