@@ -12,7 +12,7 @@
 // correctly rounded reciprocals of their divisors (dev::div_rn: the same bits;
 // operands outside its range take the division), the three divisions by one
 // length or w share one reciprocal, and the powers of the gamma are formed
-// from the hardware's base-2 logarithm and exponential (pow_pos).
+// from the hardware's base-2 logarithm and exponential (pow_pos): 36.9 us.
 //
 // Conventions (the oracle's): the pixel is sampled at its centre; the world
 // position is inverse(P*V) of the centre's NDC; the VSM is sampled
@@ -57,8 +57,10 @@ __device__ __forceinline__ float smoothstep_f(float e0, float e1, float x) {
 // x^y for x > 0 (0 otherwise), y = 2.2 or 1 / 2.2: 2^(y log2 x) with x = m 2^e,
 // m in [0.75, 1.5), so that the hardware logarithm's error is one of a value
 // below 0.6, and y e split from the sum with its rounding error before the
-// exponential takes the fraction. Within 2 ulp where the hardware functions
-// are within one; ~20 instructions.
+// exponential takes the fraction; ~20 instructions. Over all significands at 12
+// exponents the gamma is off by at most 1.03 ulp, 0.26 on average (the library's
+// powf here: 1.32 and 0.34). The same in FP64, 0.503 ulp, takes 49 us in place
+// of 37 at 1080p.
 __device__ __forceinline__ float pow_pos(float x, float y) {
   const float h = __builtin_amdgcn_frexp_mantf(x);  // [0.5, 1)
   const bool low = h < 0.75f;
@@ -70,6 +72,13 @@ __device__ __forceinline__ float pow_pos(float x, float y) {
   const float f = (p - n) + __builtin_fmaf(y, l, __builtin_fmaf(y, e, -p));
   const float r = __builtin_amdgcn_ldexpf(__builtin_amdgcn_exp2f(f), (int)n);
   return x > 0.0f ? r : 0.0f;
+}
+
+// x^20 for x >= 0: products in FP64 round once (0.51 ulp). Seen through the
+// gamma, in units of 2^-23: 0.94 at most; five products in FP32 3.76, powf 1.39.
+__device__ __forceinline__ float pow20(float x) {
+  const double x1 = (double)x, x2 = x1 * x1, x4 = x2 * x2, x5 = x4 * x1, x10 = x5 * x5;
+  return (float)(x10 * x10);
 }
 
 // shadowmapping.glsl:13-20
@@ -142,8 +151,7 @@ __global__ __launch_bounds__(256) void composite_kernel(CompositeArgs a) {
   const float dist = sqrtf(dlx * dlx + dly * dly + dlz * dlz);
   const float shadow = vsm_factor(mx, my, dist) * (sc[3] > 0.0f ? 1.0f : 0.0f);
   const float occ = a.occlusion ? a.occlusion[c] : 1.0f;
-  const float h1 = fmaxf(0.0f, ndoth), h2 = h1 * h1, h4 = h2 * h2, h5 = h4 * h1, h10 = h5 * h5;
-  const float spec_f = h10 * h10;  // (n . h)^20
+  const float spec_f = pow20(fmaxf(0.0f, ndoth));
   float res[3];
 #pragma unroll
   for (int k = 0; k < 3; ++k) {

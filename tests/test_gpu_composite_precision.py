@@ -2,7 +2,12 @@
 
 A variance shadow map cleared to a huge or infinite distance ("no occluder")
 lights, as the division by the smoothstep's window says (+inf, clamped to 1),
-and so does a variance whose reciprocal FP32 cannot hold."""
+and so does a variance whose reciprocal FP32 cannot hold. The powers are seen
+one at a time, through scenes whose other factors are exact: the gamma is
+within 1.32 ulp of the 64-bit power of its FP32 argument, which is what the
+library's powf reaches here over all significands, and (n.h)^20 within 0.51 ulp
+(half for the rounding to FP32). What passes through the gamma has its relative
+error divided by 2.2; an ulp is at most 2^-23 of its number."""
 import numpy as np
 import pytest
 
@@ -11,6 +16,9 @@ import mlgi
 pytestmark = pytest.mark.gpu
 
 F = np.float32
+GAMMA = float(F(1) / F(2.2))
+POWF = 1.32
+ULP = 2.0 ** -23
 
 
 def scene(w, h, **kw):
@@ -42,6 +50,10 @@ def run(ctx, i, p):
     return out.numpy()
 
 
+def ulps(got, want):
+    return np.abs(got.astype(np.float64) - want) / np.spacing(want.astype(F)).astype(np.float64)
+
+
 @pytest.mark.parametrize("first,second", [(1e30, np.inf), (3.5e35, np.inf), (3e38, np.inf),
                                           (np.finfo(F).max, np.finfo(F).max), (np.inf, np.inf), (0.0, 1.5e38),
                                           (0.0, 3e38), (1e18, 2e38)])
@@ -53,3 +65,25 @@ def test_huge_moments_light(ctx, first, second):
     i["vsm"][..., 0], i["vsm"][..., 1] = first, second
     assert want.min() > 0.2
     assert np.array_equal(run(ctx, i, p), want)
+
+
+def test_gamma(ctx):
+    print("[composite] gamma", flush=True)
+    rng = np.random.default_rng(3)
+    g = np.exp(rng.uniform(np.log(1e-36), np.log(1e6), (64, 512, 3))).astype(F)
+    out = run(ctx, *scene(512, 64, diffuse=np.ones_like(g), gi=g, light_intensity=0.0))
+    q = (g / (F(1) + g)).astype(np.float64)
+    assert ulps(out, q ** GAMMA).max() <= POWF
+
+
+def test_highlight(ctx):
+    print("[composite] highlight", flush=True)
+    e = np.random.default_rng(5).uniform(0.75, 1.0, (64, 512)).astype(F)
+    nz = (e * F(2) - F(1)).astype(np.float64)
+    n = np.full((64, 512, 3), 0.5, F)
+    n[..., 2] = e
+    scale = 2.0 ** -40
+    out = run(ctx, *scene(512, 64, normal=n, specular=np.ones((64, 512, 3), F), exposure=scale))
+    want = ((0.75 * nz ** 20 * scale) ** GAMMA)[..., None]
+    # the power, its product with 0.75 (half an ulp) and the gamma
+    assert (np.abs(out - want) / want).max() <= ((0.51 + 0.5) * GAMMA + POWF) * ULP
