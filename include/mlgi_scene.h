@@ -97,7 +97,10 @@ int mlgi_scene_render_surface(const mlgi_scene* s, const mlgi_camera* cam, int32
  * The scene's BVH on the device, for inputs that change per request or per
  * frame (light poses, views). The kernels run the host renderer's double
  * precision code, so their texels equal mlgi_scene_render_gbuffer /
- * mlgi_scene_render_rsm bit for bit. Output pointers are device buffers;
+ * mlgi_scene_render_rsm bit for bit, for near planes up to 2^28 times the
+ * scene's extent away (beyond, where the doubles no longer resolve the scene,
+ * either may miss a triangle). Rays that are not finite (no far plane, a camera
+ * at its own centre) hit nothing. Output pointers are device buffers;
  * the launches are asynchronous on the context stream. */
 typedef struct mlgi_scene_device mlgi_scene_device;
 int mlgi_scene_upload(mlgi_context* ctx, const mlgi_scene* s, mlgi_scene_device** out);

@@ -69,55 +69,18 @@ __device__ __forceinline__ void wave_sync() {
 
 __device__ __forceinline__ bool any_lane(bool b) { return __ballot(b) != 0ull; }
 
-// A lane's ray for the FP32 box tests: slab distances lo * i + c along each
-// axis, measured from the ray's entry into the scene's box (`entry`, 0 for a
-// ray that starts inside), and the largest distance still of interest.
-struct BoxRay {
-  float ix, iy, iz, cx, cy, cz, tmax;
-  double entry;
-};
-
-// A bound on the distance to t that is not below it (FP32 rounding, 2^-24).
-__device__ __forceinline__ float box_tmax(double t, double entry) { return (float)(t - entry) * (1.0f + 0x1p-22f); }
-
-__device__ __forceinline__ BoxRay box_ray(const SceneView& s, D3 o, D3 d, double tmax) {
-  BoxRay r;
-  r.entry = 0.0;
+// The packet's box rays: one that starts outside the scene's box is moved to
+// its entry (the margin of the scene's box covers the double rounding here).
+__device__ __forceinline__ BoxRay packet_box_ray(const SceneView& s, D3 o, D3 d, double tmax) {
   bool in = true;
-  const bool outside = !(o.x >= s.lo[0] && o.x <= s.hi[0] && o.y >= s.lo[1] && o.y <= s.hi[1] && o.z >= s.lo[2] &&
-                         o.z <= s.hi[2]);
+  double entry = 0.0;
+  const bool outside = outside_scene(s, o);
   if (any_lane(outside)) {
-    // the margin of the scene's box covers the double rounding here
     double t0;
     in = box_hit(s.lo, s.hi, o, ray_inverse(d), tmax, &t0);
-    if (outside && in) r.entry = t0;
+    if (outside && in) entry = t0;
   }
-  const D3 p = o + d * r.entry;
-  auto inverse = [](double v) {
-    const float f = (float)v;
-    return __builtin_amdgcn_rcpf(fabsf(f) < 1e-18f ? copysignf(1e-18f, f) : f);
-  };
-  r.ix = inverse(d.x);
-  r.iy = inverse(d.y);
-  r.iz = inverse(d.z);
-  r.cx = -((float)p.x * r.ix);
-  r.cy = -((float)p.y * r.iy);
-  r.cz = -((float)p.z * r.iz);
-  r.tmax = in ? box_tmax(tmax, r.entry) : -1.0f;
-  return r;
-}
-
-// Whether the ray enters the box at most r.tmax away (the distance is
-// clamped to 0 and returned). An unused child's box, a point at 1e18 on every
-// axis, is never hit: its distances are beyond any tmax or negative.
-__device__ __forceinline__ bool box_test(const BoxRay& r, float lx, float ly, float lz, float hx, float hy, float hz,
-                                         float& near) {
-  const float ax = __builtin_fmaf(lx, r.ix, r.cx), bx = __builtin_fmaf(hx, r.ix, r.cx);
-  const float ay = __builtin_fmaf(ly, r.iy, r.cy), by = __builtin_fmaf(hy, r.iy, r.cy);
-  const float az = __builtin_fmaf(lz, r.iz, r.cz), bz = __builtin_fmaf(hz, r.iz, r.cz);
-  near = fmaxf(fmaxf(fmaxf(fminf(ax, bx), fminf(ay, by)), fminf(az, bz)), 0.0f);
-  const float far = fminf(fminf(fminf(fmaxf(ax, bx), fmaxf(ay, by)), fmaxf(az, bz)), r.tmax);
-  return near <= far;
+  return box_ray(o, d, entry, tmax, in);
 }
 
 // The packet's direction octant, from its first lane: any octant orders the
@@ -155,7 +118,7 @@ __device__ Hit trace_rays(const SceneView& s, D3 o, D3 d, double tmax, PacketLds
   typedef float f8 __attribute__((ext_vector_type(8)));
   const int lane = threadIdx.x;
   Hit h{tmax, -1};
-  BoxRay r = box_ray(s, o, d, tmax);
+  BoxRay r = packet_box_ray(s, o, d, tmax);
   const int oct = packet_octant(d);
   const int pair = oct < 4 ? oct : oct ^ 7;  // the stored order; reversed for octants 4..7
   int sp = 0;
@@ -268,7 +231,7 @@ __device__ __forceinline__ uint32_t any_of_quads(unsigned long long b) {
 __device__ Hit trace_quads(const SceneView& s, D3 o, D3 d, double tmax, PacketLds<16>& lds) {
   const int lane = threadIdx.x, q = lane & 3, slot = lane >> 2;
   Hit h{tmax, -1};  // the same in a quad's lanes
-  BoxRay r = box_ray(s, o, d, tmax);
+  BoxRay r = packet_box_ray(s, o, d, tmax);
   const int oct = packet_octant(d);
   const int pair = oct < 4 ? oct : oct ^ 7;
   int sp = 0;

@@ -249,9 +249,9 @@ int collapse8(mlgi_scene* s, const std::vector<Node>& bin, int b, float margin, 
     c.after = 0;
     if (k >= n) {
       c.ref = kNoChild;
-      // a point no ray reaches: the slab test sorts each axis's two planes, so
-      // an inverted box would count as an endless one
-      for (int a = 0; a < 3; ++a) c.lo[a] = c.hi[a] = 1e18f;
+      // a point no ray reaches (box_test): the slab test sorts each axis's two
+      // planes, so an inverted box would count as an endless one
+      for (int a = 0; a < 3; ++a) c.lo[a] = c.hi[a] = HUGE_VALF;
       continue;
     }
     const Node& x = bin[kid[k]];

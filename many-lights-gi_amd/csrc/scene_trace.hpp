@@ -66,8 +66,9 @@ constexpr uint32_t kNoChild = 0xFFFFFFFFu;
 // magnitude m. A ray's FP32 slab distances are off by at most (2^-21 + 2^-22) m
 // in position along an axis: the reciprocal direction (rounded direction and
 // hardware reciprocal, 2^-22 of a distance of at most 2 m), the rounded origin
-// (2^-24 m, the origin moved into the scene's box first), its product with the
-// reciprocal (2^-24 m) and the final sum (2^-24 of 2 m).
+// (2^-24 m, the origin moved into the scene's box first: from up to 2^28 m away
+// that adds 2^-24 m), its product with the reciprocal (2^-24 m) and the final
+// sum (2^-24 of 2 m).
 constexpr float kBoxMargin = 0x1p-20f;
 
 // Triangle geometry in leaf order for the intersection test: v0 and the two
@@ -108,6 +109,67 @@ MLGI_HD inline bool box_hit(const float lo_[3], const float hi_[3], D3 o, D3 inv
   }
   *tnear = t0;
   return !(t0 > t1);
+}
+
+MLGI_HD inline D3 ray_inverse(D3 d) {
+  return {1.0 / (d.x != 0 ? d.x : 1e-300), 1.0 / (d.y != 0 ? d.y : 1e-300), 1.0 / (d.z != 0 ? d.z : 1e-300)};
+}
+
+// A ray for the packets' FP32 box tests: slab distances lo * i + c along each
+// axis, measured from the ray's entry into the scene's box (`entry`, 0 for a
+// ray that starts inside), and the largest distance still of interest.
+struct BoxRay {
+  float ix, iy, iz, cx, cy, cz, tmax;
+  double entry;
+};
+
+// A bound on the distance to t that is not below it (FP32 rounding, 2^-24).
+MLGI_HD inline float box_tmax(double t, double entry) { return (float)(t - entry) * (1.0f + 0x1p-22f); }
+
+MLGI_HD inline bool outside_scene(const SceneView& s, D3 o) {
+  return !(o.x >= s.lo[0] && o.x <= s.hi[0] && o.y >= s.lo[1] && o.y <= s.hi[1] && o.z >= s.lo[2] && o.z <= s.hi[2]);
+}
+
+// 1 / v, finite and not 0 for every v.
+MLGI_HD inline float box_inverse(double v) {
+  const float f = (float)v;
+  const float g = copysignf(fminf(fmaxf(fabsf(f), 1e-18f), 0x1p100f), f);
+#ifdef __HIP_DEVICE_COMPILE__
+  return __builtin_amdgcn_rcpf(g);
+#else
+  return 1.0f / g;
+#endif
+}
+
+MLGI_HD inline BoxRay box_ray(D3 o, D3 d, double entry, double tmax, bool in) {
+  BoxRay r;
+  r.entry = entry;
+  const D3 p = o + d * entry;
+  r.ix = box_inverse(d.x);
+  r.iy = box_inverse(d.y);
+  r.iz = box_inverse(d.z);
+  r.cx = -((float)p.x * r.ix);
+  r.cy = -((float)p.y * r.iy);
+  r.cz = -((float)p.z * r.iz);
+  // a ray that misses the scene's box, or is not finite (a camera without a far
+  // plane, or at its own centre): it enters no box and hits nothing, as on the
+  // host. tmax is compared, the distances, which may be NaN, are not.
+  const bool finite = fabsf(r.cx) < HUGE_VALF && fabsf(r.cy) < HUGE_VALF && fabsf(r.cz) < HUGE_VALF;
+  r.tmax = in && finite ? box_tmax(tmax, entry) : -1.0f;
+  return r;
+}
+
+// Whether the ray enters the box at most r.tmax away (the distance is
+// clamped to 0 and returned). An unused child's box, a point at infinity on
+// every axis, is never hit: where tmax is not negative its distances are
+// infinite (i is not 0 and c is finite) and tmax is finite.
+MLGI_HD inline bool box_test(const BoxRay& r, float lx, float ly, float lz, float hx, float hy, float hz, float& near) {
+  const float ax = __builtin_fmaf(lx, r.ix, r.cx), bx = __builtin_fmaf(hx, r.ix, r.cx);
+  const float ay = __builtin_fmaf(ly, r.iy, r.cy), by = __builtin_fmaf(hy, r.iy, r.cy);
+  const float az = __builtin_fmaf(lz, r.iz, r.cz), bz = __builtin_fmaf(hz, r.iz, r.cz);
+  near = fmaxf(fmaxf(fmaxf(fminf(ax, bx), fminf(ay, by)), fminf(az, bz)), 0.0f);
+  const float far = fminf(fminf(fminf(fmaxf(ax, bx), fmaxf(ay, by)), fmaxf(az, bz)), r.tmax);
+  return near <= far;
 }
 
 // Moller-Trumbore, two-sided, in two steps: the determinant and the three
@@ -167,10 +229,6 @@ struct LocalStack {
 // nodes in packets (raycast.hip). Which of the triangles is nearest, and which
 // of equally near ones wins, does not depend on the order of the visits, so
 // both give the same hit.
-MLGI_HD inline D3 ray_inverse(D3 d) {
-  return {1.0 / (d.x != 0 ? d.x : 1e-300), 1.0 / (d.y != 0 ? d.y : 1e-300), 1.0 / (d.z != 0 ? d.z : 1e-300)};
-}
-
 inline Hit trace(const SceneView& s, D3 o, D3 d, double tmax, LocalStack& st) {
   Hit h{tmax, -1};
   const D3 inv = ray_inverse(d);
