@@ -289,8 +289,9 @@ int collapse8(mlgi_scene* s, const std::vector<Node>& bin, int b, float margin, 
 // (only for far larger scenes than generated here), median splits and whole
 // levels: at most 7 pending children for each three binary levels, of which
 // median splits make ceil(log2(n / 4)) + 2 <= 31. Then the triangle geometry
-// in leaf order.
-void build_bvh(mlgi_scene* s) {
+// in leaf order. False where neither tree stays below `stack` pending children
+// (not for kTraceStack).
+bool build_bvh(mlgi_scene* s, int stack = kTraceStack) {
   const int n = (int)s->tris.size();
   std::vector<Prim> prims(n);
   Box scene;
@@ -318,11 +319,13 @@ void build_bvh(mlgi_scene* s) {
     s->hi[k] = round_up_f((double)scene.hi[k] + margin);
   }
   std::vector<Node> bin;
-  for (int levels = 0; levels < 2; ++levels) {
+  bool fits = false;
+  for (int levels = 0; levels < 2 && !fits; ++levels) {
     build_binary(prims, span, levels ? 0 : 64, bin);
     s->nodes.clear();
-    if (collapse8(s, bin, 0, margin, levels != 0) < kTraceStack) break;
+    fits = collapse8(s, bin, 0, margin, levels != 0) < stack;
   }
+  if (!fits) return false;
   s->order.resize(n);
   s->geo.assign(n + kGeoPad, TriGeo{});
   for (int i = 0; i < n; ++i) {
@@ -330,6 +333,7 @@ void build_bvh(mlgi_scene* s) {
     const Tri& t = s->tris[s->order[i]];
     s->geo[i] = TriGeo{t.v0, t.v1 - t.v0, t.v2 - t.v0};
   }
+  return true;
 }
 
 // 4x4 column-major helpers in double
@@ -486,7 +490,10 @@ int mlgi_scene_create(uint64_t seed, int32_t n_random, mlgi_scene** out) {
     ++made;
   }
   for (const Tri& t : s->tris) s->area += 0.5 * len(cross(t.v1 - t.v0, t.v2 - t.v0));
-  build_bvh(s);
+  if (!build_bvh(s)) {
+    delete s;
+    return MLGI_ERR_UNSUPPORTED;
+  }
   *out = s;
   return MLGI_OK;
 }
