@@ -325,12 +325,11 @@ struct TileJob {
 // the eight L2s, which the end of the kernel waits for. Write-through stores
 // (agent scope, sc1) go to memory as they are issued and leave the atlas in the
 // last-level cache for the pull-push: 1080p frame 187.0 -> 185.7 us, splat and
-// pull-push of a 2,048^2 atlas 45.4 -> 43.5. From kStreamBytes of atlas in a
-// launch on it would have left that cache (256 MB) before the pull-push comes;
+// pull-push of a 2,048^2 atlas 45.4 -> 43.5. From 176 MiB of atlas in a launch on
+// (tiles_stream) it would have left that cache (256 MB) before the pull-push comes;
 // stored as a stream (nt) it does not push the points and masks out either.
 // Write-through / stream, us: batches with 68 MB of tiles 201/203, 132 MB
 // 262/270, 196 MB 381/370, 329 MB 582/557, 403 MB 814/776.
-constexpr uint64_t kStreamBytes = uint64_t(176) << 20;
 constexpr int kAuxStream = 2, kAuxWriteThrough = 16;  // nt, sc1
 
 template <int kAux>
@@ -659,7 +658,7 @@ hipError_t launch_ism_splat_tiled(hipStream_t s, const float* points, const uint
     if (e != hipSuccess) return e;
   }
   const int n_tiles = n1d * n1d;
-  const bool stream = (uint64_t)n_tiles * ism_side * ism_side * 4 >= kStreamBytes;
+  const bool stream = tiles_stream((uint64_t)n_tiles * ism_side * ism_side * 4);
   const dim3 grid(xcd_items_grid((uint32_t)n_tiles));
   if (ism_side > 32)
     hipLaunchKernelGGL(ism_tiles_kernel<uint16_t>, grid, dim3(256), tile_lds_bytes<uint16_t>(ism_side), s, j, n_tiles,
@@ -704,11 +703,12 @@ hipError_t launch_batch_mask(hipStream_t s, const BatchFrame* frames, int n, uin
   return hipGetLastError();
 }
 
-hipError_t launch_batch_tiles(hipStream_t s, const BatchFrame* frames, int n, uint32_t total, int max_side) {
+hipError_t launch_batch_tiles(hipStream_t s, const BatchFrame* frames, int n, uint32_t total, int max_side,
+                              uint64_t bytes) {
   if (total == 0) return hipSuccess;
   if (max_side < 4 || max_side > kTileMax) return hipErrorInvalidValue;
   const dim3 grid(xcd_items_grid(total));
-  const bool stream = (uint64_t)total * max_side * max_side * 4 >= kStreamBytes;
+  const bool stream = tiles_stream(bytes);
   if (max_side > 32)
     hipLaunchKernelGGL(batch_tiles_kernel<uint16_t>, grid, dim3(256), tile_lds_bytes<uint16_t>(max_side), s, frames, n,
                        total, max_side, stream);

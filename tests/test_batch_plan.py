@@ -1,0 +1,38 @@
+"""What a batch's plan tells its launches (CPU only, no device): the tile pass
+streams its stores from 176 MiB of tiles on, counted over the frames' own
+atlases, whatever the largest ISM side among them."""
+import ctypes as C
+import subprocess
+from pathlib import Path
+
+import pytest
+
+import mlgi
+
+SRC = Path(__file__).with_name("batch_plan.cpp")
+MIB = 1 << 20
+
+
+@pytest.fixture(scope="module")
+def lib(tmp_path_factory):
+    so = tmp_path_factory.mktemp("plan") / "libplan.so"
+    native = Path(mlgi.__file__).parent
+    subprocess.run(["g++", "-O1", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
+                    str(SRC), "-o", str(so), f"-L{native}", "-l:libmlgi.so", f"-Wl,-rpath,{native}"], check=True)
+    return C.CDLL(str(so))
+
+
+@pytest.mark.parametrize("frames,mib,stream", [
+    ([(4096, 4096)] + [(1024, 1024)] * 8, 96, False),  # ISMs of 64^2 beside 32^2
+    ([(256, 1024)] + [(4096, 1024)] * 30, 124, False),  # of 64^2 beside 16^2
+    ([(4096, 4096)] * 2 + [(4096, 2048)] * 3, 176, True),
+    ([(1024, 1024)] * 43, 172, False),
+    ([(1024, 1024)] * 44, 176, True),
+])
+def test_tile_bytes(lib, frames, mib, stream):
+    n = len(frames)
+    vpl, side = ((C.c_int * n)(*c) for c in zip(*frames))
+    total, largest = C.c_uint64(0), C.c_int(0)
+    assert lib.plan_tiles(n, vpl, side, C.byref(total), C.byref(largest)) == 0
+    assert total.value == mib * MIB
+    assert bool(lib.streams(total)) == stream
