@@ -167,13 +167,6 @@ class Copier {
   std::vector<std::thread> threads_;
 };
 
-// Pinned staging per batch slot for results on their way to the callers'
-// memory. A copy to pageable memory blocks the host until the batch's stream
-// has run dry, so no other batch is admitted or retired meanwhile; a copy to
-// pinned memory is queued (a burst of 24 requests: 4.25 ms direct, 2.36 ms
-// staged). At most this much per slot and in all; results that do not fit go
-// directly, as all do where no memory can be pinned.
-constexpr size_t kStageSlotBytes = size_t(16) << 20, kStageBytes = size_t(96) << 20;
 constexpr int kCopyHelpers = 3;
 
 struct GBuf {
@@ -277,7 +270,7 @@ struct mlgi_server {
   // batch tables: ring of max_queued_batches slots of max_batch rows
   mlgi::BatchFrame* table_dev = nullptr;
   mlgi::BatchFrame* table_host = nullptr;  // pinned
-  char* stage = nullptr;                   // pinned, stage_bytes per slot
+  char* stage = nullptr;                   // pinned, stage_bytes per slot (stage_slot_bytes)
   size_t stage_bytes = 0;
   std::unique_ptr<Copier> copier;
   std::vector<hipEvent_t> events;
@@ -480,8 +473,7 @@ int mlgi_server_create(mlgi_context* c, const mlgi_server_config* cfg, const mlg
   if (!rc) {
     size_t largest = 0;
     for (auto& wh : s->resolutions) largest = std::max(largest, (size_t)wh.first * wh.second * 12);
-    s->stage_bytes = std::min(kStageSlotBytes, kStageBytes / (size_t)cfg->max_queued_batches);
-    s->stage_bytes = std::min(s->stage_bytes, largest * (size_t)cfg->max_batch);
+    s->stage_bytes = stage_slot_bytes(cfg->max_queued_batches, largest, cfg->max_batch);
     if (hipHostMalloc((void**)&s->stage, s->stage_bytes * cfg->max_queued_batches, hipHostMallocDefault) !=
         hipSuccess) {
       (void)hipGetLastError();
@@ -639,7 +631,7 @@ int mlgi_server_run(mlgi_server* s, const mlgi_request* reqs, int32_t n, mlgi_se
             if (may_stage[a.req] && used + bytes <= s->stage_bytes) {
               staged.push_back({dst, stage + used, bytes});
               dst = stage + used;
-              used += bytes;
+              used += stage_round(bytes);
             }
             rc = hip_check(c, hipMemcpyAsync(dst, a.image, bytes, hipMemcpyDeviceToHost, L->stream),
                            "hipMemcpyAsync(result)");

@@ -1,4 +1,4 @@
-// Plans of batches without a device, for tests/test_batch_plan.py (linked with
+// Plans of batches and of a server's staging without a device, for tests/test_batch_plan.py (linked with
 // libmlgi.so).
 #include "../include/mlgi_scene.h"
 
@@ -41,6 +41,10 @@ extern "C" int plan_tiles(int n, const int* vpl, const int* side, uint64_t* byte
   *bytes = plan.tile_bytes;
   *max_side = plan.max_ism_side;
   return rc;
+}
+
+extern "C" size_t stage_slot(int slots, size_t largest, int max_batch) {
+  return mlgi_capi::stage_slot_bytes(slots, largest, max_batch);
 }
 
 extern "C" int streams(uint64_t bytes) { return mlgi::tiles_stream(bytes); }

@@ -1,6 +1,7 @@
 """What a batch's plan tells its launches (CPU only, no device): the tile pass
 streams its stores from 176 MiB of tiles on, counted over the frames' own
-atlases, whatever the largest ISM side among them."""
+atlases, whatever the largest ISM side among them; a server's staging slots
+start on 256-byte lines for every number of slots."""
 import ctypes as C
 import subprocess
 from pathlib import Path
@@ -36,3 +37,13 @@ def test_tile_bytes(lib, frames, mib, stream):
     assert lib.plan_tiles(n, vpl, side, C.byref(total), C.byref(largest)) == 0
     assert total.value == mib * MIB
     assert bool(lib.streams(total)) == stream
+
+
+def test_stage_slots_are_aligned(lib):
+    lib.stage_slot.argtypes, lib.stage_slot.restype = [C.c_int, C.c_size_t, C.c_int], C.c_size_t
+    for slots in range(1, 65):
+        for largest in (17 * 9 * 12, 1917 * 1079 * 12, 16384 * 16384 * 12):
+            for batch in (1, 7, 32):
+                b = lib.stage_slot(slots, largest, batch)
+                assert b % 256 == 0 and b * slots <= 96 * MIB and b <= 16 * MIB
+                assert b >= min(largest * batch, 16 * MIB, 96 * MIB // slots - 255)
