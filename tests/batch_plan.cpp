@@ -47,4 +47,8 @@ extern "C" size_t stage_slot(int slots, size_t largest, int max_batch) {
   return mlgi_capi::stage_slot_bytes(slots, largest, max_batch);
 }
 
+extern "C" int pp_group(int ism_side, int isms, int frames) {
+  return mlgi::pullpush_group(ism_side, (uint64_t)isms * frames, isms);
+}
+
 extern "C" int streams(uint64_t bytes) { return mlgi::tiles_stream(bytes); }

@@ -1,7 +1,8 @@
 """What a batch's plan tells its launches (CPU only, no device): the tile pass
 streams its stores from 176 MiB of tiles on, counted over the frames' own
 atlases, whatever the largest ISM side among them; a server's staging slots
-start on 256-byte lines for every number of slots."""
+start on 256-byte lines for every number of slots; and the pull-push takes the
+groups of ISMs that test_gpu_pullpush_groups.py means to run."""
 import ctypes as C
 import subprocess
 from pathlib import Path
@@ -9,6 +10,7 @@ from pathlib import Path
 import pytest
 
 import mlgi
+from test_gpu_pullpush_groups import BATCHES, SINGLE
 
 SRC = Path(__file__).with_name("batch_plan.cpp")
 MIB = 1 << 20
@@ -47,3 +49,11 @@ def test_stage_slots_are_aligned(lib):
                 b = lib.stage_slot(slots, largest, batch)
                 assert b % 256 == 0 and b * slots <= 96 * MIB and b <= 16 * MIB
                 assert b >= min(largest * batch, 16 * MIB, 96 * MIB // slots - 255)
+
+
+def test_pullpush_groups(lib):
+    assert {g for *_, g in SINGLE} == {4, 16, 64} == {g for *_, g in BATCHES}
+    for side, n1d, group in SINGLE:
+        assert lib.pp_group(side, n1d * n1d, 1) == group
+    for side, n1d, frames, group in BATCHES:
+        assert lib.pp_group(side, n1d * n1d, frames) == group
