@@ -349,7 +349,8 @@ typedef struct mlgi_frame_desc {
   mlgi_rsm rsm;
   mlgi_points points;
   mlgi_gbuffer gbuffer;
-  mlgi_params params;   /* per frame; tile_w selects the gather strip width (8, 16, 32) */
+  mlgi_params params;   /* per frame; tile_w selects the gather's strips, one wave each: 8 x 8, 16 x 4
+                           or 32 x 2 pixels of a class (8 x 8 also for a 16 x 16 tile that shadows) */
   mlgi_vpls vpls;       /* caller-owned work and output buffers */
   mlgi_atlas atlas;
   mlgi_ism_depth ism;   /* must not overlap the atlas, as for mlgi_ism_pullpush */
@@ -376,9 +377,11 @@ void mlgi_batch_destroy(mlgi_batch* batch);
  *   interleave: the largest of {8, 4} that leaves at least
  *     min_vpls_per_pixel VPLs per interleave class (else 4); it decides
  *     which VPLs a pixel sums, i.e. the image, so it follows a quality rule;
- *   tile: the fastest gather strip width of {8, 16, 32} (workgroup tiles
- *     8x8, 16x4 / 16x16, 32x8), timed on the frame itself through the batch
- *     path; the image does not depend on it.
+ *   tile: the fastest batched gather strip of {8 x 8, 16 x 4, 32 x 2}, timed
+ *     on the frame itself through the batch path and written as the tiles 8x8,
+ *     16x4 and 32x8 (a single-frame 32x8 tile runs as waves of 8 x 8, so for
+ *     mlgi_frame its time is near the 8x8 tile's); the image does not depend
+ *     on it.
  * Writes the choice into frame->params (interleave, use_interleaving,
  * tile_w, tile_h). Results are cached per shape in the context; a cached
  * shape is not timed again. Runs the frame (its buffers are overwritten). */

@@ -1016,7 +1016,8 @@ int batch_frame(mlgi_context* c, const mlgi_frame_desc& d, mlgi::BatchFrame* f) 
   a.ism = d.ism.texels;  // the pull-push writes it even when the gather does not shadow
   f->g = a;
   // a 16 x 16 tile is four 8 x 8 waves where it shadows, as in the
-  // single-frame kernel
+  // single-frame kernel; a width of 32 stays the strip of 32 x 2 that the
+  // autotuner times against the 8 x 8 ones
   const int wave_w = tw == 16 && p->tile_h == 16 && a.shadowing ? 8 : tw;
   f->wave_w_log2 = log2i(wave_w);
   const int cw = (a.width + a.interleave - 1) / a.interleave;

@@ -734,7 +734,7 @@ hipError_t launch_batch_gather(hipStream_t s, const BatchFrame* frames, int n, u
   const unsigned grid = (unsigned)((total + per_round - 1) / per_round * per_round);
   if (precision == 1)
     hipLaunchKernelGGL(batch_gather_kernel<true>, dim3(grid), dim3(64), 0, s, frames, n, total, chunk_log2);
-  else if (ahead_pays(false, true, total))
+  else if (ahead_pays(false, true, total))  // a batch may mix both kinds: the lower line
     hipLaunchKernelGGL(batch_gather_ahead_kernel, dim3(grid), dim3(64), 0, s, frames, n, total, chunk_log2);
   else
     hipLaunchKernelGGL(batch_gather_kernel<false>, dim3(grid), dim3(64), 0, s, frames, n, total, chunk_log2);

@@ -579,11 +579,11 @@ constexpr int level_offset(int l) {  // texels of pull levels 1..l-1 of one ISM
   return o;
 }
 
-// ISMs per workgroup: as many S x S ISMs as make 64^2 texels (1 at S = 64,
-// 4 at 32, 16 at 16, 64 at 8), so that the small levels of several ISMs share
-// wave iterations (a level of one output costs a full wave iteration per
-// workgroup). At most the frame's ISM count; both are powers of four, so the
-// group divides it.
+// Most ISMs per workgroup, which size the LDS: as many S x S ISMs as make 64^2
+// texels (1 at S = 64, 4 at 32, 16 at 16, 64 at 8), so that the small levels of
+// several ISMs share wave iterations (a level of one output costs a full wave
+// iteration per workgroup). A launch takes what pullpush_group says: fewer
+// while it has under 512 workgroups.
 template <int S>
 constexpr int kGroupMax = (64 / S) * (64 / S);
 
